@@ -138,38 +138,44 @@ hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid
 // *ppCount, zeroed by the caller) and limited by launch_pp_lanes.
 // la (Euler, may be null): the learned WENO selection runs in the same kernel
 // on the staged brick (outputs those of launch_learned_select).
+// PW (Euler, may be null): the parity coefficients of the face points
+// (host/parity.hpp, [type][C]) of mirror-symmetric weights; without them
+// the dense products with W0T.
 hipError_t launch_linear(int dim, int nq, int nv, const double *U, double *FS, double *WI,
                          double *thetaNew, const double *props, const Grid &g, const double *W0,
-                         const double *W0T, int *ppList, int *ppCount, hipStream_t s,
-                         const LearnArgs *la = nullptr);
+                         const double *W0T, int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la,
+                         const double *PW);
 // Euler: the limiter's exact sequence on the cells of launch_linear whose
 // states failed the fast test (list, size *count); those wflag marks for
 // WENO are skipped.
 hipError_t launch_pp_lanes(int dim, int nq, const double *U, double *FS, double *thetaNew,
                            const double *props, const double *wflag, const Grid &g,
                            const int *list, const int *count, hipStream_t s);
-// ---- fused path of the Euler equations in sparse mode.  Rows: the listed
+// ---- fused path of the Euler equations in sparse mode (mirror-symmetric
+// weights; fused_flux: the shapes it is built for).  With the 9 points per face
+// of the 3D 3x3 rule a thread would hold 90 states of an axis; those run the
+// unfused kernels.  Rows: the listed
 // cells' limited face states, row t = [F*Q*5] (WENO cells at their list
 // positions, then the cells of the limiter's exact sequence), pos[cell] = the
 // cell's row or -1.
+constexpr bool fused_flux(int dim, int nq) { return dim == 2 || nq == 2; }
 // Surface planes for the grid (doubles; fills sb).
 size_t surf_elems(int dim, int nq, const Grid &g, Surf &sb);
 // Linear reconstruction with the fast limiter test (slow cells to ppList, the
 // others get theta 1) and the KXRCF indicator (WI may be null), storing only
 // the states on brick-boundary faces, into SB.
 hipError_t launch_linear_surf(int dim, int nq, const double *U, double *WI, double *thetaNew,
-                              const double *props, const Grid &g, const double *W0T, int *ppList, int *ppCount,
-                              double *SB, const Surf &sb, hipStream_t s);
+                              const double *props, const Grid &g, const double *PW, int *ppList, int *ppCount,
+                              double *SB, const Surf &sb, hipStream_t s, const LearnArgs *la);
 // The limiter's exact sequence on the slow cells of launch_linear_surf not
 // marked for WENO: recomputed linear states, limited, into rows
 // *wenoCount + 0, 1, ... (counted in *rowCount, zeroed by the caller).
 hipError_t launch_pp_rows(int dim, int nq, const double *U, double *rows, int *pos, double *thetaNew,
-                          const double *props, const double *wflag, const Grid &g, const double *W0,
+                          const double *props, const double *wflag, const Grid &g, const double *PW,
                           const int *list, const int *count, const int *wenoCount, int *rowCount, hipStream_t s);
-// Linear states of the cells without a row (recomputed, weights WQ
-// [Q][C][F]), rows of the others, SB across brick boundaries; Riemann solves,
+// Linear states of the cells without a row (recomputed), rows of the others, SB across brick boundaries; Riemann solves,
 // divergence and the RK epilogue of launch_flux_rk.
-hipError_t launch_flux_fused(int dim, int nq, const double *U, const double *WQ, const double *rows, const int *pos,
+hipError_t launch_flux_fused(int dim, int nq, const double *U, const double *PW, const double *rows, const int *pos,
                              const double *SB, const Surf &sb, const Grid &g, const RKArgs &a, hipStream_t s);
 // pos (may be null): per-cell list position below cap, -1 otherwise
 hipError_t launch_select(int dim, int nq, const double *U, const double *WI, const double *theta,
@@ -242,6 +248,10 @@ hipError_t launch_mhd_chmax(int dim, const double *spd, const Grid &g, unsigned 
 // 3D: 0 = 16x4x4); the partial count follows it.
 hipError_t launch_flux_rk(int dim, int nq, int nv, const double *U, const double *FS,
                           const Grid &g, const RKArgs &a, hipStream_t s, int shape = 0);
+// The same for 3D Euler runs with the learned selection, in their order of
+// operations (points5.hpp).
+hipError_t launch_flux_points(int dim, int nq, const double *U, const double *FS, const Grid &g, const RKArgs &a,
+                              hipStream_t s);
 int flux_rk_partials(int dim, const Grid &g, int shape = 0);
 // Batch of slices: per-slice finalize (out[2 s], out[2 s + 1]) over the flux
 // kernel's blocks, which are slice-major (blocksPerSlice each), and the copy of

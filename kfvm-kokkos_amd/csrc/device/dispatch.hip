@@ -6,14 +6,15 @@
 
 namespace kfvm {
 
-#define KFVM_SELECT(dim, nq, CALL)                          \
+#define KFVM_SELECT_OF(LAUNCH, dim, nq, CALL)               \
   do {                                                      \
-    if (dim == 3 && nq == 2) { using L = Launch<3, 2>; return CALL; } \
-    if (dim == 3 && nq == 3) { using L = Launch<3, 3>; return CALL; } \
-    if (dim == 2 && nq == 2) { using L = Launch<2, 2>; return CALL; } \
-    if (dim == 2 && nq == 3) { using L = Launch<2, 3>; return CALL; } \
+    if (dim == 3 && nq == 2) { using L = LAUNCH<3, 2>; return CALL; } \
+    if (dim == 3 && nq == 3) { using L = LAUNCH<3, 3>; return CALL; } \
+    if (dim == 2 && nq == 2) { using L = LAUNCH<2, 2>; return CALL; } \
+    if (dim == 2 && nq == 3) { using L = LAUNCH<2, 3>; return CALL; } \
     return hipErrorInvalidValue;                            \
   } while (0)
+#define KFVM_SELECT(dim, nq, CALL) KFVM_SELECT_OF(Launch, dim, nq, CALL)
 
 hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s) {
   KFVM_SELECT(dim, 2, L::cell_props(U, props, g, s));
@@ -21,25 +22,26 @@ hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid
 
 hipError_t launch_linear(int dim, int nq, int nv, const double *U, double *FS, double *WI,
                          double *thetaNew, const double *props, const Grid &g, const double *W0,
-                         const double *W0T, int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la) {
+                         const double *W0T, int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la,
+                         const double *PW) {
   if (nv != 5 && nv != 1) return hipErrorInvalidValue;
   if (la && nv != 5) return hipErrorInvalidValue;
-  KFVM_SELECT(dim, nq, L::linear(nv, U, FS, WI, thetaNew, props, g, W0, W0T, ppList, ppCount, s, la));
+  KFVM_SELECT(dim, nq, L::linear(nv, U, FS, WI, thetaNew, props, g, W0, W0T, ppList, ppCount, s, la, PW));
 }
 
 hipError_t launch_linear_surf(int dim, int nq, const double *U, double *WI, double *thetaNew,
-                              const double *props, const Grid &g, const double *W0T, int *ppList, int *ppCount,
-                              double *SB, const Surf &sb, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::linear_surf(U, WI, thetaNew, props, g, W0T, ppList, ppCount, SB, sb, s));
+                              const double *props, const Grid &g, const double *PW, int *ppList, int *ppCount,
+                              double *SB, const Surf &sb, hipStream_t s, const LearnArgs *la) {
+  KFVM_SELECT(dim, nq, L::linear_surf(U, WI, thetaNew, props, g, PW, ppList, ppCount, SB, sb, s, la));
 }
 hipError_t launch_pp_rows(int dim, int nq, const double *U, double *rows, int *pos, double *thetaNew,
-                          const double *props, const double *wflag, const Grid &g, const double *W0,
+                          const double *props, const double *wflag, const Grid &g, const double *PW,
                           const int *list, const int *count, const int *wenoCount, int *rowCount, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::pp_rows(U, rows, pos, thetaNew, props, wflag, g, W0, list, count, wenoCount, rowCount, s));
+  KFVM_SELECT(dim, nq, L::pp_rows(U, rows, pos, thetaNew, props, wflag, g, PW, list, count, wenoCount, rowCount, s));
 }
-hipError_t launch_flux_fused(int dim, int nq, const double *U, const double *WQ, const double *rows, const int *pos,
+hipError_t launch_flux_fused(int dim, int nq, const double *U, const double *PW, const double *rows, const int *pos,
                              const double *SB, const Surf &sb, const Grid &g, const RKArgs &a, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::flux_fused(U, WQ, rows, pos, SB, sb, g, a, s));
+  KFVM_SELECT(dim, nq, L::flux_fused(U, PW, rows, pos, SB, sb, g, a, s));
 }
 size_t surf_elems(int dim, int nq, const Grid &g, Surf &sb) {
   const int q = dim == 3 ? nq * nq : nq;
@@ -94,28 +96,28 @@ hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double
 }
 
 hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s) {
-  KFVM_SELECT(dim, 2, L::mhd_props(U, props, g, s));
+  KFVM_SELECT_OF(LaunchMhd, dim, 2, L::props(U, props, g, s));
 }
 hipError_t launch_mhd_linear(int dim, int nq, const double *U, double *FS, double *SRC, double *WI,
                              double *thetaNew, double *spd, const double *props, const Grid &g, const double *WT,
                              int *ppList, int *ppCount, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::mhd_linear(U, FS, SRC, WI, thetaNew, spd, props, g, WT, ppList, ppCount, s));
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::linear(U, FS, SRC, WI, thetaNew, spd, props, g, WT, ppList, ppCount, s));
 }
 hipError_t launch_mhd_select(int dim, int nq, const double *U, const double *WI, const double *theta,
                              double *wflag, int *list, int *counter, double wThresh, const Grid &g,
                              hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::mhd_select(U, WI, theta, wflag, list, counter, wThresh, g, s));
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::select(U, WI, theta, wflag, list, counter, wThresh, g, s));
 }
 hipError_t launch_mhd_weno(int dim, int nq, const double *U, double *FS, double *SRC, const Grid &g,
                            const double *FT, const double *DT, const double *CT, const int *list,
                            const int *counter, double *thetaNew, double *spd, const double *props,
                            const double *WC, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::mhd_weno(U, FS, SRC, g, FT, DT, CT, list, counter, thetaNew, spd, props, WC, s));
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::weno(U, FS, SRC, g, FT, DT, CT, list, counter, thetaNew, spd, props, WC, s));
 }
 hipError_t launch_mhd_pp(int dim, int nq, const double *U, double *FS, double *SRC, double *thetaNew,
                          double *spd, const double *props, const double *wflag, const Grid &g, const int *list,
                          const int *count, hipStream_t s) {
-  KFVM_SELECT(dim, nq, L::mhd_pp(U, FS, SRC, thetaNew, spd, props, wflag, g, list, count, s));
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::pp(U, FS, SRC, thetaNew, spd, props, wflag, g, list, count, s));
 }
 hipError_t launch_flow_stats(int dim, int nv, const double *U, const Grid &g, double ifac, double *out,
                             hipStream_t s) {
@@ -133,7 +135,13 @@ hipError_t launch_flux_rk(int dim, int nq, int nv, const double *U, const double
                           const Grid &g, const RKArgs &a, hipStream_t s, int shape) {
   if (nv != 5 && nv != 1 && nv != 9) return hipErrorInvalidValue;
   if (shape < 0 || shape > (dim == 2 ? 2 : 0)) return hipErrorInvalidValue;
+  if (nv == 9) KFVM_SELECT_OF(LaunchMhd, dim, nq, L::flux_rk(U, FS, g, a, s, shape));
   KFVM_SELECT(dim, nq, L::flux_rk(nv, U, FS, g, a, s, shape));
+}
+
+hipError_t launch_flux_points(int dim, int nq, const double *U, const double *FS, const Grid &g, const RKArgs &a,
+                              hipStream_t s) {
+  KFVM_SELECT(dim, nq, L::flux_points(U, FS, g, a, s));
 }
 
 int flux_rk_partials(int dim, const Grid &g, int shape) {

@@ -27,13 +27,20 @@ hipError_t Launch<D, NQ>::cell_props(const double *U, double *props, const Grid 
 template <int D, int NQ>
 hipError_t Launch<D, NQ>::linear(int nv, const double *U, double *FS, double *WI, double *thetaNew,
                                  const double *props, const Grid &g, const double *W0, const double *W0T,
-                                 int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la) {
-  if (nv == 5 && la)
-    hipLaunchKernelGGL((dev::k_linear_fused<D, NQ, false, true>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s,
-                       U, FS, WI, thetaNew, props, g, W0T, ppList, ppCount, nullptr, Surf{}, *la);
+                                 int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la, const double *PW) {
+  const dim3 nb(bricks(g)), nt(dev::RBox<D>::NT);
+  if (nv == 5 && PW && la)
+    hipLaunchKernelGGL((dev::k_linear_par<D, NQ, false, true>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, PW,
+                       ppList, ppCount, nullptr, Surf{}, *la);
+  else if (nv == 5 && PW)
+    hipLaunchKernelGGL((dev::k_linear_par<D, NQ, false, false>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, PW,
+                       ppList, ppCount, nullptr, Surf{}, LearnArgs{});
+  else if (nv == 5 && la)
+    hipLaunchKernelGGL((dev::k_linear_fused<D, NQ, true>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, W0T, ppList,
+                       ppCount, *la);
   else if (nv == 5)
-    hipLaunchKernelGGL((dev::k_linear_fused<D, NQ>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U, FS, WI,
-                       thetaNew, props, g, W0T, ppList, ppCount);
+    hipLaunchKernelGGL((dev::k_linear_fused<D, NQ, false>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, W0T, ppList,
+                       ppCount, LearnArgs{});
   else
     hipLaunchKernelGGL((dev::k_linear<D, NQ, 1>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, FS, WI,
                        thetaNew, g, W0);
@@ -80,29 +87,49 @@ hipError_t Launch<D, NQ>::weno(int nv, const double *U, double *FS, double *thet
 
 template <int D, int NQ>
 hipError_t Launch<D, NQ>::linear_surf(const double *U, double *WI, double *thetaNew, const double *props,
-                                      const Grid &g, const double *W0T, int *ppList, int *ppCount, double *SB,
-                                      const Surf &sb, hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_linear_fused<D, NQ, true>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U,
-                     nullptr, WI, thetaNew, props, g, W0T, ppList, ppCount, SB, sb);
-  return hipGetLastError();
+                                      const Grid &g, const double *PW, int *ppList, int *ppCount, double *SB,
+                                      const Surf &sb, hipStream_t s, const LearnArgs *la) {
+  if constexpr (fused_flux(D, NQ)) {
+    const dim3 nb(bricks(g)), nt(dev::RBox<D>::NT);
+    if (la)
+      hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, true>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g,
+                         PW, ppList, ppCount, SB, sb, *la);
+    else
+      hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, false>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g,
+                         PW, ppList, ppCount, SB, sb, LearnArgs{});
+    return hipGetLastError();
+  } else {
+    return hipErrorInvalidValue;
+  }
 }
 
 template <int D, int NQ>
 hipError_t Launch<D, NQ>::pp_rows(const double *U, double *rows, int *pos, double *thetaNew, const double *props,
-                                  const double *wflag, const Grid &g, const double *W0, const int *list,
+                                  const double *wflag, const Grid &g, const double *PW, const int *list,
                                   const int *count, const int *wenoCount, int *rowCount, hipStream_t s) {
-  const unsigned np = std::min<unsigned>(stage_blocks(g.ncell), 4096u);
-  hipLaunchKernelGGL((dev::k_pp_rows<D, NQ>), dim3(np), dim3(dev::BLK), 0, s, U, rows, pos, thetaNew, props,
-                     wflag, g, W0, list, count, wenoCount, rowCount);
-  return hipGetLastError();
+  if constexpr (fused_flux(D, NQ)) {
+    const unsigned np = std::min<unsigned>(stage_blocks(g.ncell), 4096u);
+    hipLaunchKernelGGL((dev::k_pp_rows<D, NQ>), dim3(np), dim3(dev::BLK), 0, s, U, rows, pos, thetaNew, props,
+                       wflag, g, PW, list, count, wenoCount, rowCount);
+    return hipGetLastError();
+  } else {
+    return hipErrorInvalidValue;
+  }
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::flux_fused(const double *U, const double *WQ, const double *rows, const int *pos,
+hipError_t Launch<D, NQ>::flux_fused(const double *U, const double *PW, const double *rows, const int *pos,
                                      const double *SB, const Surf &sb, const Grid &g, const RKArgs &a, hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_flux_fused<D, NQ>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U, WQ, rows, pos,
-                     SB, sb, g, a);
-  return hipGetLastError();
+  if constexpr (fused_flux(D, NQ)) {
+    const dim3 nb(bricks(g)), nt(dev::RBox<D>::NT);
+    if (g.rs == 2)
+      hipLaunchKernelGGL((dev::k_flux_par<D, NQ, true>), nb, nt, 0, s, U, PW, rows, pos, SB, sb, g, a);
+    else
+      hipLaunchKernelGGL((dev::k_flux_par<D, NQ, false>), nb, nt, 0, s, U, PW, rows, pos, SB, sb, g, a);
+    return hipGetLastError();
+  } else {
+    return hipErrorInvalidValue;
+  }
 }
 
 template <int D, int NQ>
@@ -129,30 +156,30 @@ hipError_t Launch<D, NQ>::weno_post(const double *U, double *FS, double *thetaNe
 }
 
 template <int D, int NQ>
-unsigned Launch<D, NQ>::mhd_bricks(const Grid &g) {
+unsigned LaunchMhd<D, NQ>::bricks(const Grid &g) {
   using Bx = dev::MBox<D>;
   return unsigned(((g.nx + Bx::BX - 1) / Bx::BX) * ((g.ny + Bx::BY - 1) / Bx::BY) *
                   ((g.nz + Bx::BZ - 1) / Bx::BZ));
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::mhd_props(const double *U, double *props, const Grid &g, hipStream_t s) {
+hipError_t LaunchMhd<D, NQ>::props(const double *U, double *props, const Grid &g, hipStream_t s) {
   hipLaunchKernelGGL((dev::k_mhd_props<D>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, props, g);
   return hipGetLastError();
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::mhd_linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew,
+hipError_t LaunchMhd<D, NQ>::linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew,
                                      double *spd, const double *props, const Grid &g, const double *WT,
                                      int *ppList, int *ppCount, hipStream_t s) {
   // WI null: the learned selection does not read the KXRCF indicator
-  hipLaunchKernelGGL((dev::k_mhd_linear<D, NQ>), dim3(mhd_bricks(g)), dim3(dev::MBox<D>::NT), 0, s, U, FS, SRC,
+  hipLaunchKernelGGL((dev::k_mhd_linear<D, NQ>), dim3(bricks(g)), dim3(dev::MBox<D>::NT), 0, s, U, FS, SRC,
                      WI, thetaNew, spd, props, g, WT, ppList, ppCount);
   return hipGetLastError();
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::mhd_select(const double *U, const double *WI, const double *theta, double *wflag,
+hipError_t LaunchMhd<D, NQ>::select(const double *U, const double *WI, const double *theta, double *wflag,
                                      int *list, int *counter, double wThresh, const Grid &g, hipStream_t s) {
   hipLaunchKernelGGL((dev::k_select<D, NQ, dev::Mhd>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, WI,
                      theta, wflag, list, counter, wThresh, g, nullptr, 0);
@@ -160,7 +187,7 @@ hipError_t Launch<D, NQ>::mhd_select(const double *U, const double *WI, const do
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::mhd_weno(const double *U, double *FS, double *SRC, const Grid &g, const double *FT,
+hipError_t LaunchMhd<D, NQ>::weno(const double *U, double *FS, double *SRC, const Grid &g, const double *FT,
                                    const double *DT, const double *CT, const int *list, const int *counter,
                                    double *thetaNew, double *spd, const double *props, const double *WC,
                                    hipStream_t s) {
@@ -181,7 +208,7 @@ hipError_t Launch<D, NQ>::mhd_weno(const double *U, double *FS, double *SRC, con
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::mhd_pp(const double *U, double *FS, double *SRC, double *thetaNew, double *spd,
+hipError_t LaunchMhd<D, NQ>::pp(const double *U, double *FS, double *SRC, double *thetaNew, double *spd,
                                  const double *props, const double *wflag, const Grid &g, const int *list,
                                  const int *count, hipStream_t s) {
   const unsigned np = std::min<unsigned>(stage_blocks(g.ncell), 1024u);
@@ -274,27 +301,54 @@ dim3 Launch<D, NQ>::flux_grid(const Grid &g, int shape) {
   return count(dev::Brick<D, 0>{});
 }
 
-template <int D, int NQ>
-hipError_t Launch<D, NQ>::flux_rk(int nv, const double *U, const double *FS, const Grid &g, const RKArgs &a,
-                                  hipStream_t s, int shape) {
-  auto run = [&](auto shp) {
-    constexpr int S = decltype(shp)::value;
-    using Bk = dev::Brick<D, S>;
-    const dim3 blk(Bk::X, Bk::Y, Bk::Z);
-    if (nv == 5)
-      hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 5, S>), flux_grid(g, S), blk, 0, s, U, FS, g, a);
-    else if (nv == 9)
-      hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 9, S>), flux_grid(g, S), blk, 0, s, U, FS, g, a);
-    else
-      hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 1, S>), flux_grid(g, S), blk, 0, s, U, FS, g, a);
-    return hipGetLastError();
-  };
+// Calls run(shape constant) for the brick shape of a flux launch.
+template <int D, class F>
+hipError_t with_shape(int shape, F &&run) {
   if constexpr (D == 2) {
     if (shape == 1) return run(std::integral_constant<int, 1>{});
     if (shape == 2) return run(std::integral_constant<int, 2>{});
   }
   if (shape != 0 && D == 3) return hipErrorInvalidValue;
   return run(std::integral_constant<int, 0>{});
+}
+
+template <int D, int NQ>
+hipError_t Launch<D, NQ>::flux_rk(int nv, const double *U, const double *FS, const Grid &g, const RKArgs &a,
+                                  hipStream_t s, int shape) {
+  return with_shape<D>(shape, [&](auto shp) {
+    constexpr int S = decltype(shp)::value;
+    using Bk = dev::Brick<D, S>;
+    const dim3 blk(Bk::X, Bk::Y, Bk::Z);
+    if (nv == 5)
+      hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 5, S>), flux_grid(g, S), blk, 0, s, U, FS, g, a);
+    else
+      hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 1, S>), flux_grid(g, S), blk, 0, s, U, FS, g, a);
+    return hipGetLastError();
+  });
+}
+
+template <int D, int NQ>
+hipError_t Launch<D, NQ>::flux_points(const double *U, const double *FS, const Grid &g, const RKArgs &a,
+                                      hipStream_t s) {
+  if constexpr (D == 3) {
+    using Bk = dev::Brick<D>;
+    hipLaunchKernelGGL((dev::k_flux_points<NQ>), flux_grid(g, 0), dim3(Bk::X, Bk::Y, Bk::Z), 0, s, U, FS, g, a);
+    return hipGetLastError();
+  } else {
+    return hipErrorInvalidValue;
+  }
+}
+
+template <int D, int NQ>
+hipError_t LaunchMhd<D, NQ>::flux_rk(const double *U, const double *FS, const Grid &g, const RKArgs &a,
+                                     hipStream_t s, int shape) {
+  return with_shape<D>(shape, [&](auto shp) {
+    constexpr int S = decltype(shp)::value;
+    using Bk = dev::Brick<D, S>;
+    hipLaunchKernelGGL((dev::k_flux_rk<D, NQ, 9, S>), (Launch<D, NQ>::flux_grid(g, S)), dim3(Bk::X, Bk::Y, Bk::Z), 0,
+                       s, U, FS, g, a);
+    return hipGetLastError();
+  });
 }
 
 }  // namespace kfvm

@@ -53,6 +53,23 @@ __device__ inline double sqrt_n(double x) {
   g = fma(fma(-g, g, x), h, g);
   return x == 0.0 ? x : g;  // rsq(0) = inf
 }
+// sqrt_n of an operand known to be nonzero
+__device__ inline double sqrt_nz(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = fma(-g, h, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  g = fma(fma(-g, g, x), h, g);
+  return fma(fma(-g, g, x), h, g);
+}
+// 1 / sqrt(x): the estimate, one Goldschmidt step and one Newton step
+__device__ inline double rsqrt_n(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  const double g = x * y, h = 0.5 * y;
+  y = fma(y, fma(-g, h, 0.5), y);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
 // a / b and sqrt(x), the IEEE operations or (N) the sequences above
 template <bool N>
 __device__ inline double dv(double a, double b) {
@@ -134,12 +151,87 @@ struct Hydro {
     return sMax;
   }
   // HLLC with the low-Mach / shear corrections (Hydro_Riemann.H:97-187).  The
-  // formulas are the reference's; divisions by a common denominator are
+  // formulas are the reference's, arranged for few divisions and square roots,
+  // which are most of the solver's time (each takes 8 to 16 issue slots):
+  //   - a common denominator is inverted once; 1/rho of both sides comes from
+  //     the reciprocal of their product;
+  //   - the larger of |v_L|/a_L and |v_R|/a_R is picked by its square, so M takes
+  //     one reciprocal square root instead of two roots and two divisions;
+  //   - the star state is formed on the side the face lies on only;
+  //   - the pressure ratio enters the power without being divided out
+  //     (pow_ratio).
+  // 4 reciprocals, 2 quotients and 7 roots, against 5, 6 and 8 in solve_hllc_pt.
+  // Results differ from the reference's by rounding only.
+  template <int DIR>
+  __device__ static inline double solve_hllc(double g, const double *uL, const double *uR,
+                                             double *F) {
+    constexpr int v0 = 1 + DIR, v1 = 1 + (DIR + 1) % 3, v2 = 1 + (DIR + 2) % 3;
+    const double gm1 = g - 1.0;
+    const double rhoL = uL[0], rhoR = uR[0];
+    const double ir = rcp_n(rhoL * rhoR), irL = ir * rhoR, irR = ir * rhoL;
+    const double unL = uL[v0] * irL, vtL = uL[v1] * irL, wtL = uL[v2] * irL;
+    const double unR = uR[v0] * irR, vtR = uR[v1] * irR, wtR = uR[v2] * irR;
+    const double vsqL = unL * unL + vtL * vtL + wtL * wtL, vsqR = unR * unR + vtR * vtR + wtR * wtR;
+    const double pL = gm1 * (uL[4] - 0.5 * rhoL * vsqL), pR = gm1 * (uR[4] - 0.5 * rhoR * vsqR);
+    const double aaL = g * pL * irL, aaR = g * pR * irR;  // a^2
+    const double aL = sqrt_n(aaL), aR = sqrt_n(aaR);
+    const double hL = (uL[4] + pL) * irL, hR = (uR[4] + pR) * irR;
+    // Batten speeds from Roe averages
+    const double srL = sqrt_nz(rhoL), srR = sqrt_nz(rhoR), iS = rcp_n(srL + srR);
+    const double uTil = (unL * srL + unR * srR) * iS, vTil = (vtL * srL + vtR * srR) * iS;
+    const double wTil = (wtL * srL + wtR * srR) * iS, hTil = (hL * srL + hR * srR) * iS;
+    const double vsqTil = uTil * uTil + vTil * vTil + wTil * wTil;
+    const double aTil = sqrt_n(gm1 * (hTil - 0.5 * vsqTil));
+    const double sL = fmin(unL - aL, uTil - aTil), sR = fmax(unR + aR, uTil + aTil);
+    const double sMax = fmax(fabs(sL), fabs(sR));
+    // M = max(|v|/a) over the sides with a real sound speed
+    const bool mL = aaL >= 0.0 && (!(aaR >= 0.0) || !(vsqL * aaR <= vsqR * aaL));
+    const double mNum = mL ? vsqL : vsqR, mDen = mL ? aaL : aaR;
+    double M = mNum == 0.0 ? 0.0 : mNum * rsqrt_n(mNum * mDen);
+    const double psL0 = rhoL * (sL - unL), psR0 = rhoR * (sR - unR);
+    const double dPs = psL0 - psR0, iPs = rcp_n(dPs), nS = (pR - pL) + (psL0 * unL - psR0 * unR);
+    double sS = nS * iPs;
+    sS = fma(fma(-dPs, sS, nS), iPs, sS);
+    const double pS = 0.5 * ((pL + pR) + psL0 * (sS - unL) + psR0 * (sS - unR));
+    const double uJump = unR - unL, vJump = vtR - vtL, wJump = wtR - wtL;
+    const double psiFac = -(psR0 * psL0) * iPs;
+    const bool pLow = pL < pR;
+    const double gFac = 1.0 - pow_ratio(pLow ? pL : pR, pLow ? pR : pL, M);  // M >= 0
+    M = fmin(M, 1.0);
+    const double oneMsq = 1.0 - M * M;
+    const double fM = div_n(M * sqrt_nz(4.0 + oneMsq * oneMsq), 1.0 + M * M);
+    // regions of the reference: 0 <= sL: F(uL); else 0 <= sS: star L;
+    // else 0 < sR: star R; else F(uR)
+    const bool left = 0.0 <= sL || 0.0 <= sS;
+    double u[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) u[v] = left ? uL[v] : uR[v];
+    const double un = left ? unL : unR, vt = left ? vtL : vtR, wt = left ? wtL : wtR;
+    const double p = left ? pL : pR;
+    F[0] = u[v0];
+    F[v0] = u[v0] * un + p;
+    F[v1] = u[v0] * vt;
+    F[v2] = u[v0] * wt;
+    F[4] = un * (u[4] + p);
+    const double sK = left ? sL : sR, iK = rcp_n(sK - sS);
+    if (left ? !(0.0 <= sL) : 0.0 < sR) {
+      const double sFac = sS * iK, sI = sK * iK;
+      const double shFac = psiFac * gFac * sI, pFac = psiFac * (fM - 1.0) * uJump + pS * sI;
+      F[0] = sFac * (sK * u[0] - F[0]);
+      F[v0] = sFac * (sK * u[v0] - F[v0]) + pFac;
+      F[v1] = sFac * (sK * u[v1] - F[v1]) + shFac * vJump;
+      F[v2] = sFac * (sK * u[v2] - F[v2]) + shFac * wJump;
+      F[4] = sFac * (sK * u[4] - F[4]) + sS * pFac;
+    }
+    return sMax;
+  }
+  // The same solver with both sides' star factors formed (k_flux_points, whose
+  // results are reproduced bit for bit).  The formulas are the reference's; divisions by a common denominator are
   // multiplications by its reciprocal (10 divisions instead of 29), and the
   // divisions and square roots are rcp_n / div_n / sqrt_n, so results differ
   // from the reference's by rounding only.
   template <int DIR>
-  __device__ static inline double solve_hllc(double g, const double *uL, const double *uR,
+  __device__ static inline double solve_hllc_pt(double g, const double *uL, const double *uR,
                                              double *F) {
     constexpr int v0 = 1 + DIR, v1 = 1 + (DIR + 1) % 3, v2 = 1 + (DIR + 2) % 3;
     const double gm1 = g - 1.0;

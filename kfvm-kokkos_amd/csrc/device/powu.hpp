@@ -21,18 +21,12 @@
 
 namespace kfvm {
 
-KFVM_POWU_HD inline double powu(double x, double y) {
-  if (!(x > 0.0)) return x == 0.0 ? (y > 0.0 ? 0.0 : 1.0) : x;  // 0^y; NaN passes through
+// exp(y (e ln 2 + 2 atanh s))
+KFVM_POWU_HD inline double exp_y_ln(double s, int e, double y) {
   constexpr double LN2_HEAD = 0.6931467056274414;      // ln 2 with 32 trailing zero bits
   constexpr double LN2_TAIL = 4.7493250390316726e-07;  // ln 2 - LN2_HEAD
   constexpr double INV_LN2 = 1.4426950408889634;
-  int e;
-  double m = std::frexp(x, &e);
-  if (m < 0.70710678118654752) {
-    m *= 2.0;
-    e -= 1;
-  }
-  const double s = (m - 1.0) / (m + 1.0), s2 = s * s;
+  const double s2 = s * s;
   double p = 1.0 / 23.0;
   p = std::fma(p, s2, 1.0 / 21.0);
   p = std::fma(p, s2, 1.0 / 19.0);
@@ -65,6 +59,47 @@ KFVM_POWU_HD inline double powu(double x, double y) {
   q = std::fma(q, r, 1.0);
   q = std::fma(q, r, 1.0);
   return std::ldexp(q, int(n));
+}
+
+KFVM_POWU_HD inline double powu(double x, double y) {
+  if (!(x > 0.0)) return x == 0.0 ? (y > 0.0 ? 0.0 : 1.0) : x;  // 0^y; NaN passes through
+  int e;
+  double m = std::frexp(x, &e);
+  if (m < 0.70710678118654752) {
+    m *= 2.0;
+    e -= 1;
+  }
+  return exp_y_ln((m - 1.0) / (m + 1.0), e, y);
+}
+
+// (a/b)^y for 0 <= a <= b, b > 0 and y >= 0: as powu, with the ratio taken
+// inside the logarithm, a = m 2^ea, b = n 2^eb, m/n brought into [1/sqrt 2,
+// sqrt 2), s = (m-n)/(m+n): one division less than powu(a / b, y), and no
+// rounding of the ratio (tests/test_pow_ratio.py: the bounds of powu).
+#ifdef __HIPCC__
+namespace dev {
+__device__ inline double div_n(double a, double b);  // physics.hpp
+}
+#endif
+
+KFVM_POWU_HD inline double pow_ratio(double a, double b, double y) {
+  if (!(a > 0.0)) return a == 0.0 ? (y > 0.0 ? 0.0 : 1.0) : a / b;  // 0^y; NaN passes through
+  int ea, eb;
+  double m = std::frexp(a, &ea);
+  const double n = std::frexp(b, &eb);
+  int e = ea - eb;
+  if (m < 0.70710678118654752 * n) {
+    m *= 2.0;
+    e -= 1;
+  } else if (m > 1.4142135623730951 * n) {
+    m *= 0.5;
+    e += 1;
+  }
+#ifdef __HIP_DEVICE_COMPILE__
+  return exp_y_ln(dev::div_n(m - n, m + n), e, y);
+#else
+  return exp_y_ln((m - n) / (m + n), e, y);
+#endif
 }
 
 }  // namespace kfvm

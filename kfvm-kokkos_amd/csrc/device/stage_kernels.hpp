@@ -29,7 +29,10 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 
+#include "../host/parity.hpp"
 #include "../host/stencil_geom.hpp"
 #include "device_api.hpp"
 #include "physics.hpp"
@@ -518,21 +521,43 @@ __global__ __launch_bounds__(BLK) void k_weno(const double *__restrict__ U,
 }
 
 // -------------------------------------------- Riemann + divergence + RK update
-template <int NV, int DIR>
-__device__ inline double riemann(const Grid &g, double ch, const double *uL, const double *uR,
+// Conserved variable at position v once the momenta (and the field) are
+// rotated cyclically so that the component along axis dir comes first.  One
+// solver serves the three directions: a third of the solver code, which for
+// GLM-MHD did not fit the instruction cache three times over.
+template <int NV>
+__device__ inline int rotated_var(int v, int dir) {
+  const bool mom = NV >= 5 && v >= 1 && v <= 3, fld = NV == 9 && v >= 5 && v <= 7;
+  if (!mom && !fld) return v;
+  const int first = mom ? 1 : 5, r = v - first + dir;
+  return first + (r >= 3 ? r - 3 : r);
+}
+
+// Quadrature weight of face point q (selects: an indexed load of the Grid
+// argument would put it in scratch).
+template <int D, int NQ>
+__device__ inline double face_weight(const Grid &g, int q) {
+  auto w = [&](int n) { return n == 0 ? g.wt[0] : (n == 1 ? g.wt[1] : g.wt[2]); };
+  return D == 2 ? w(q) : w(q / NQ) * w(q % NQ);
+}
+
+// Flux and fastest wave of one face along axis dir from the rotated states of
+// its two sides (rotated_var); the flux comes back rotated the same way.
+template <int NV>
+__device__ inline double riemann(const Grid &g, int dir, double ch, const double *uL, const double *uR,
                                  double *Fl) {
   if (NV == 9) {
-    if (g.rs == 4) return Mhd::solve_kepes<DIR>(g.gamma, ch, uL, uR, Fl);
-    return Mhd::solve_hll<DIR>(g.gamma, ch, g.rs == 0, uL, uR, Fl);
+    if (g.rs == 4) return Mhd::solve_kepes<0>(g.gamma, ch, uL, uR, Fl);
+    return Mhd::solve_hll<0>(g.gamma, ch, g.rs == 0, uL, uR, Fl);
   } else if (NV == 5) {
-    if (g.rs == 2) return Hydro::solve_hllc<DIR>(g.gamma, uL, uR, Fl);
-    return Hydro::solve_hll<DIR>(g.gamma, g.rs == 0, uL, uR, Fl);
+    if (g.rs == 2) return Hydro::solve_hllc<0>(g.gamma, uL, uR, Fl);
+    return Hydro::solve_hll<0>(g.gamma, g.rs == 0, uL, uR, Fl);
   } else {
-    if (!g.haveVel && DIR == 2) {
+    if (!g.haveVel && dir == 2) {
       Fl[0] = 0.0;
       return 0.0;
     }
-    const double a = g.vel[DIR];
+    const double a = dir == 0 ? g.vel[0] : (dir == 1 ? g.vel[1] : g.vel[2]);
     Fl[0] = a > 0.0 ? a * uL[0] : a * uR[0];
     return fabs(a);
   }
@@ -704,20 +729,15 @@ __device__ void mhd_source_rhs(const double *__restrict__ U, const double *__res
                                double *rhs);
 
 template <int D, int NQ, int NV, int S = 0>
-__global__ __launch_bounds__(BLK) void k_flux_rk(const double *__restrict__ U,
+__global__ __launch_bounds__(BLK, NV == 9 ? (D == 3 && NQ == 3 ? 1 : 2) : 3) void k_flux_rk(const double *__restrict__ U,
                                                  const double *__restrict__ FS, Grid g,
                                                  RKArgs a) {
   using Bk = Brick<D, S>;
   constexpr int Q = Shape<D, NQ>::Q;
   __shared__ double fl[NV][Bk::NF];
-  // GLM-MHD: normal field averaged over the two states of each face (div B)
+  // GLM-MHD: normal field averaged over the two states of each face point,
+  // integrated over the face (div B)
   __shared__ double bvf[NV == 9 ? Bk::NF : 1];
-  // GLM-MHD: this cell's div B terms of each face point (x, y, z), summed
-  // after the face loop in the source kernel's point order
-  constexpr int QT = NV == 9 ? Q : 1;
-  double divT[QT][3];
-#pragma unroll
-  for (int qq = 0; qq < QT; qq++) divT[qq][0] = divT[qq][1] = divT[qq][2] = 0.0;
   // compact WENO rows of the brick's cells and their face neighbours (Euler
   // sparse WENO; -1: states in FS)
   constexpr int RX = Bk::X + 2, RY = Bk::Y + 2, RZ = D == 3 ? Bk::Z + 2 : 1;
@@ -774,15 +794,9 @@ __global__ __launch_bounds__(BLK) void k_flux_rk(const double *__restrict__ U,
     return NV == 5 ? rowTab[e] : -1;
   };
 
-  // Face items (the same for every face point q): d0 = t | dir << 20 |
-  // needed << 30 (-1: padding), and for each side the source of its states:
-  // a cell index (>= 0, its FS slots), a compact WENO row r (-(r + 2)), or the
-  // mirror of the other side (-1: a wall).  Euler and linear advection
-  // resolve them once per brick into LDS (each thread reads back only the
-  // items it wrote); GLM-MHD, whose flux planes leave no LDS for them at two
-  // workgroups per CU, resolves them at every point.
-  constexpr bool FDL = NV != 9;
-  __shared__ int fd0[FDL ? Bk::PF : 1], fdL[FDL ? Bk::PF : 1], fdR[FDL ? Bk::PF : 1];
+  // Face items: d0 = t | dir << 20 | needed << 30 (-1: padding), and for each
+  // side the source of its states: a cell index (>= 0, its FS slots), a compact
+  // WENO row r (-(r + 2)), or the mirror of the other side (-1: a wall).
   constexpr int MIRROR = -1;
   auto describe = [&](int w, int &d0, int &sL, int &sR) {
     // padded work item w -> face t of the unpadded numbering (x, then y, then z faces)
@@ -834,7 +848,9 @@ __global__ __launch_bounds__(BLK) void k_flux_rk(const double *__restrict__ U,
       const int row = row_of(x, y, z);
       if (pos < 0 || pos >= n_ax) {
         const bool low = pos < 0;
-        if ((low ? g.bc[2 * dir] : g.bc[2 * dir + 1]) != 0) return MIRROR;
+        const int bLo = dir == 0 ? g.bc[0] : (dir == 1 ? g.bc[2] : g.bc[4]);
+        const int bHi = dir == 0 ? g.bc[1] : (dir == 1 ? g.bc[3] : g.bc[5]);
+        if ((low ? bLo : bHi) != 0) return MIRROR;
         pos = low ? pos + n_ax : pos - n_ax;
         if (dir == 0) x = pos;
         else if (dir == 1) y = pos;
@@ -849,132 +865,93 @@ __global__ __launch_bounds__(BLK) void k_flux_rk(const double *__restrict__ U,
     }
     d0 = t | (dir << 20) | (needed ? 1 << 30 : 0);
   };
-  if constexpr (FDL) {
-    for (int w = tid; w < Bk::PF; w += BLK) describe(w, fd0[w], fdL[w], fdR[w]);
-  }
-  // states of face f at point q from a side's source
-  auto load_side = [&](int src, int f, int q, double *out) {
+  // states of face f at point q from a side's source, with the vectors rotated
+  // so that the face normal comes first (rot: plane of each rotated variable)
+  auto load_side = [&](int src, int f, int q, const int (&rot)[NV], double *out) {
     if (NV == 5 && src <= -2) {
       const double *r = a.ws + size_t(-src - 2) * (Shape<D, NQ>::F * Q * 5) + (f * Q + q) * 5;
 #pragma unroll
-      for (int v = 0; v < NV; v++) out[v] = r[v];
+      for (int v = 0; v < NV; v++) out[v] = r[rot[v]];
     } else {
       const double *p = FS + fs_base(size_t(src), Shape<D, NQ>::F * Q * NV) + size_t(f * Q + q) * NV * FSB;
 #pragma unroll
-      for (int v = 0; v < NV; v++) out[v] = p[size_t(v) * FSB];
+      for (int v = 0; v < NV; v++) out[v] = p[size_t(rot[v]) * FSB];
     }
   };
-  auto mirror_of = [&](const double *inner, unsigned m, double *out) {
+  auto mirror_of = [&](const double *inner, unsigned m, const int (&rot)[NV], double *out) {
     const unsigned mm = NV >= 5 ? m : 0u;
 #pragma unroll
-    for (int v = 0; v < NV; v++) out[v] = ((mm >> v) & 1u) ? -inner[v] : inner[v];
+    for (int v = 0; v < NV; v++) out[v] = ((mm >> rot[v]) & 1u) ? -inner[v] : inner[v];
   };
 
+  // Every face of the brick, solved once: a thread takes a face through all its
+  // points and keeps the flux integrated over the face in registers, so that a
+  // face is resolved once, only the integral crosses LDS and the block meets
+  // one barrier.  256^3, NQ = 2, HLLC: 5.8 ms against 6.3 with a barrier pair per
+  // point and the point fluxes in LDS; 96^3 GLM-MHD (LLF) 0.65 against 0.69.
 #pragma unroll 1
-  for (int q = 0; q < Q; q++) {
-    // every face of the brick at point q, solved once
-#pragma unroll 1
-    for (int w = tid; w < Bk::PF; w += BLK) {
-      int d0, sL, sR;
-      if constexpr (FDL) {
-        d0 = fd0[w];
-        sL = fdL[w];
-        sR = fdR[w];
-      } else {
-        describe(w, d0, sL, sR);
-      }
-      if (d0 < 0) continue;
-      const int t = d0 & 0xFFFFF, dir = (d0 >> 20) & 3;
-      double Fl[NV];
+  for (int w = tid; w < Bk::PF; w += BLK) {
+    int d0, sL, sR;
+    describe(w, d0, sL, sR);
+    if (d0 < 0) continue;
+    // the work items of a wave share their direction (padded to whole waves)
+    const int t = d0 & 0xFFFFF, dir = __builtin_amdgcn_readfirstlane((d0 >> 20) & 3);
+    int rot[NV];
 #pragma unroll
-      for (int v = 0; v < NV; v++) Fl[v] = 0.0;
-      double bv = 0.0;
-      if (d0 >> 30) {
-        double uL[NV], uR[NV];
-        const int lo = 2 * dir + 1, hi = 2 * dir;  // left cell's upper face, right cell's lower face
+    for (int v = 0; v < NV; v++) rot[v] = rotated_var<NV>(v, dir);
+    double Fs[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) Fs[v] = 0.0;
+    double bs = 0.0;
+    if (d0 >> 30) {
+      const int lo = 2 * dir + 1, hi = 2 * dir;  // left cell's upper face, right cell's lower face
+      const unsigned mLo = dir == 0 ? g.negmask[0] : (dir == 1 ? g.negmask[2] : g.negmask[4]);
+      const unsigned mHi = dir == 0 ? g.negmask[1] : (dir == 1 ? g.negmask[3] : g.negmask[5]);
+#pragma unroll 1
+      for (int q = 0; q < Q; q++) {
+        double uL[NV], uR[NV], Fl[NV];
         if (sR != MIRROR) {
-          load_side(sR, hi, q, uR);
-          if (sL == MIRROR) mirror_of(uR, g.negmask[2 * dir], uL);
-          else load_side(sL, lo, q, uL);
+          load_side(sR, hi, q, rot, uR);
+          if (sL == MIRROR) mirror_of(uR, mLo, rot, uL);
+          else load_side(sL, lo, q, rot, uL);
         } else {
-          load_side(sL, lo, q, uL);
-          mirror_of(uL, g.negmask[2 * dir + 1], uR);
+          load_side(sL, lo, q, rot, uL);
+          mirror_of(uL, mHi, rot, uR);
         }
-        double sp;
-        if (dir == 0) {
-          sp = riemann<NV, 0>(g, ch, uL, uR, Fl);
-          if constexpr (NV == 9) bv = 0.5 * (uL[5] + uR[5]);
-        } else if (dir == 1) {
-          sp = riemann<NV, 1>(g, ch, uL, uR, Fl);
-          if constexpr (NV == 9) bv = 0.5 * (uL[6] + uR[6]);
-        } else {
-          sp = riemann<NV, 2>(g, ch, uL, uR, Fl);
-          if constexpr (NV == 9) bv = 0.5 * (uL[7] + uR[7]);
-        }
+        const double wq = face_weight<D, NQ>(g, q);
+        const double sp = riemann<NV>(g, dir, ch, uL, uR, Fl);
+        if constexpr (NV == 9) bs += wq * (0.5 * (uL[5] + uR[5]));
         vmax = sp > vmax ? sp : vmax;
-      }
 #pragma unroll
-      for (int v = 0; v < NV; v++) fl[v][t] = Fl[v];
-      if constexpr (NV == 9) bvf[t] = bv;
-    }
-    __syncthreads();
-    if (live) {
-      const int tx = threadIdx.x, ty = threadIdx.y, tz = threadIdx.z;
-      const int xW = tx + (Bk::X + 1) * (ty + Bk::Y * tz), xE = xW + 1;
-      const int yS = Bk::NXF + tx + Bk::X * (ty + (Bk::Y + 1) * tz), yN = yS + Bk::X;
-      const int zB = Bk::NXF + Bk::NYF + tx + Bk::X * (ty + Bk::Y * tz), zT = zB + Bk::X * Bk::Y;
-      // the reference divides each term by the spacing; multiplying by its
-      // reciprocal differs by rounding only and saves 12 NV divisions
-      if (D == 2) {
-        const double w = g.wt[q];
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-          rhs[v] += w * (fl[v][xW] - fl[v][xE]) * rdx;
-          rhs[v] += w * (fl[v][yS] - fl[v][yN]) * rdy;
-        }
-      } else {
-        const double w = g.wt[q / NQ] * g.wt[q % NQ];
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-          rhs[v] += w * (fl[v][xW] - fl[v][xE]) * rdx;
-          rhs[v] += w * (fl[v][yS] - fl[v][yN]) * rdy;
-          rhs[v] += w * (fl[v][zB] - fl[v][zT]) * rdz;
-        }
-      }
-      if constexpr (NV == 9) {
-        // div B terms of point q as SourceTerms_K forms them (the face's
-        // average is the same from either side: the sum commutes)
-        const double twt = D == 2 ? g.wt[q] : g.wt[q % NQ] * g.wt[q / NQ];
-        const double tx = twt * (bvf[xE] - bvf[xW]) / g.dx;
-        const double ty = twt * (bvf[yN] - bvf[yS]) / g.dy;
-        const double tz = D == 3 ? twt * (bvf[zT] - bvf[zB]) / g.dz : 0.0;
-#pragma unroll
-        for (int qq = 0; qq < QT; qq++) {
-          divT[qq][0] = q == qq ? tx : divT[qq][0];
-          divT[qq][1] = q == qq ? ty : divT[qq][1];
-          divT[qq][2] = q == qq ? tz : divT[qq][2];
-        }
+        for (int v = 0; v < NV; v++) Fs[v] += wq * Fl[v];
       }
     }
-    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NV; v++) fl[rot[v]][t] = Fs[v];
+    if constexpr (NV == 9) bvf[t] = bs;
   }
-
-  if constexpr (NV == 9) {
-    if (live) {
-    // div B in the order of SourceTerms_K's point loop (MHD_GLM_K.H:316-547),
-    // then the source terms at the interior points, integrated (IntegrateRHS_K)
-    constexpr int NZ = D == 3 ? NQ : 1;
-    double divB = 0.0;
+  __syncthreads();
+  if (live) {
+    const int tx = threadIdx.x, ty = threadIdx.y, tz = threadIdx.z;
+    const int xW = tx + (Bk::X + 1) * (ty + Bk::Y * tz), xE = xW + 1;
+    const int yS = Bk::NXF + tx + Bk::X * (ty + (Bk::Y + 1) * tz), yN = yS + Bk::X;
+    const int zB = Bk::NXF + Bk::NYF + tx + Bk::X * (ty + Bk::Y * tz), zT = zB + Bk::X * Bk::Y;
+    // the reference divides each point's term by the spacing; integrating over
+    // the face first and multiplying by the reciprocal differs by rounding only
 #pragma unroll
-    for (int nQ = 0; nQ < NQ; nQ++)
-#pragma unroll
-      for (int nS = 0; nS < NZ; nS++) {
-        const int q = nS * NQ + nQ;
-        divB += divT[q][0];
-        divB += divT[q][1];
-        if (D == 3) divB += divT[q][2];
-      }
-    mhd_source_rhs<D, NQ>(U, FS, a.src, a.theta, g, a.Dm, c, ci, cj, ck, divB, rhs);
+    for (int v = 0; v < NV; v++) {
+      rhs[v] = (fl[v][xW] - fl[v][xE]) * rdx;
+      rhs[v] += (fl[v][yS] - fl[v][yN]) * rdy;
+      if (D == 3) rhs[v] += (fl[v][zB] - fl[v][zT]) * rdz;
+    }
+    if constexpr (NV == 9) {
+      // div B of SourceTerms_K (MHD_GLM_K.H:316-547) from the face integrals
+      // (a face's average is the same from either side: the sum commutes), then
+      // the source terms at the interior points, integrated (IntegrateRHS_K)
+      double divB = (bvf[xE] - bvf[xW]) * rdx;
+      divB += (bvf[yN] - bvf[yS]) * rdy;
+      if (D == 3) divB += (bvf[zT] - bvf[zB]) * rdz;
+      mhd_source_rhs<D, NQ>(U, FS, a.src, a.theta, g, a.Dm, c, ci, cj, ck, divB, rhs);
     }
   }
   const bool write = !a.sliceWrite || a.sliceWrite[slice] != 0;
@@ -996,7 +973,8 @@ __global__ __launch_bounds__(BLK) void k_flux_rk(const double *__restrict__ U,
 }  // namespace kfvm
 
 #include "recon5.hpp"
-#include "fused5.hpp"
+#include "parity5.hpp"
+#include "points5.hpp"
 #include "mhd.hpp"
 #include "indicator.hpp"
 

@@ -20,6 +20,7 @@
 #include <rocprofiler-sdk-roctx/roctx.h>
 
 #include "problems.hpp"
+#include "parity.hpp"
 #include "stencil_geom.hpp"
 
 namespace kfvm {
@@ -144,24 +145,12 @@ void Solver::setup() {
   if (rk_.needsTmp()) Utmp_ = dalloc<double>(nc * nv_, "Utmp");
   FS_ = dalloc<double>(fs_elems(nc, int(FQ) * nv_), "face states");
   if (nv_ == 5) {
-    // The linear pass stores every face state and a compact WENO staging
-    // holds the WENO states of up to a quarter of the cells, unless
-    // KFVM_FUSED=1 selects the fused reconstruction + flux path (the flux
-    // kernel recomputes the linear states from its brick: at 256^3 it costs
-    // 12.6 ms against 7.2 ms for the unfused flux kernel while the linear
-    // pass stays at 5.3 ms, since both kernels are bound by FP64 VALU work,
-    // not by the face-state traffic)
+    // Sparse mode runs the fused reconstruction + flux path where it is built
+    // and the weights are mirror-symmetric (KFVM_FUSED=0: the unfused one).
     const char *ev = std::getenv("KFVM_FUSED");
-    fused_ = ev && std::string(ev) == "1";
+    fusedWanted_ = fused_flux(cfg_.dim, cfg_.nQuad) && !(ev && std::string(ev) == "0");
     pos_ = dalloc<int>(nc, "row of each cell");
-    if (fused_) {
-      wsCap_ = int(nc);  // every listed cell has a row, in FS_
-      SB_ = dalloc<double>(surf_elems(cfg_.dim, cfg_.nQuad, grid_, sb_), "surface planes");
-      faceWQ_ = dalloc<double>(size_t(wts_.F) * wts_.Q * wts_.C, "face weights (point-major)");
-    } else {
-      wsCap_ = int(std::max<size_t>(1, (nc + 3) / 4));
-      WS_ = dalloc<double>(size_t(wsCap_) * FQ * nv_, "compact WENO states");
-    }
+    parW_ = dalloc<double>(size_t(parity_face_types(cfg_.dim, cfg_.nQuad)) * wts_.C, "parity weights");
   }
   WI_ = dalloc<double>(fs_elems(nc, int(FQ)), "indicator");
   props_ = dalloc<double>(nc * 2, "cell properties");
@@ -195,9 +184,11 @@ void Solver::setup() {
     const size_t cellRows = nv_ == 9 ? size_t(wts_.nqCell) : 0;
     faceWC_ = dalloc<double>(size_t(SUB) * (FQ + wts_.I + cellRows), "WENO weights (compact)");
   }
+  // blocks of the flux kernels: the unfused one's brick shape, the fused one's bricks
   nPart_ = flux_rk_partials(cfg_.dim, grid_, cfg_.fluxBrick);
-  errPart_ = dalloc<double>(nPart_, "err partials");
-  posPart_ = dalloc<double>(nPart_, "pos partials");
+  const int nPartMax = std::max(nPart_, flux_rk_partials(cfg_.dim, grid_, 0));
+  errPart_ = dalloc<double>(size_t(nPartMax), "err partials");
+  posPart_ = dalloc<double>(size_t(nPartMax), "pos partials");
   redOut_ = dalloc<double>(2, "reduction");
   vmax_ = dalloc<unsigned long long>(size_t(slices_), "vmax");
   if (slices_ > 1) {
@@ -405,7 +396,6 @@ int Solver::takeStepSlices() {
   int status = ACCEPTED;
   stateInCur_ = false;
   stagePos_ = 0;
-  const int blocksPerSlice = nPart_ / S;
   const bool hydro = nv_ == 5;
   // slices accepted in this step, and slices whose next evaluation runs WENO
   // on every cell (after an unphysical attempt)
@@ -481,7 +471,7 @@ int Solver::takeStepSlices() {
         a.sliceWrite = sMask_;
         pipeline(U_[cur_], a);
       }
-      check(launch_finalize_slices(errPart_, posPart_, blocksPerSlice, S, sRed_, stream_), "finalize");
+      check(launch_finalize_slices(errPart_, posPart_, nPart_ / S, S, sRed_, stream_), "finalize");
       check(hipMemcpyAsync(hRed, sRed_, 2 * size_t(S) * sizeof(double), hipMemcpyDeviceToHost, stream_), "read");
       check(hipMemcpyAsync(hVm, vmax_, size_t(S) * sizeof(double), hipMemcpyDeviceToHost, stream_), "read vmax");
       check(hipMemcpyAsync(&hostRed_[3], counter_, sizeof(int), hipMemcpyDeviceToHost, stream_), "read count");
@@ -604,7 +594,7 @@ void Solver::release() noexcept {
   } catch (...) {
   }
   void *bufs[] = {SRC_, cellW_, cellWS_, diffM_, chBits_, U_[0], U_[1], Uprev_, Uhat_, K_, Utmp_, FS_, WI_, props_, theta_[0], theta_[1], wflag_, list_, counter_, ppList_,
-                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, redOut_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, faceWQ_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
+                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, redOut_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
   if (stream_) (void)hipStreamSynchronize(stream_);
   for (auto &kv : graphs_)
     if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
@@ -740,82 +730,78 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
     timed("cell_props", [&] { return launch_cell_props(dim, Uin, props_, grid_, stream_); });
   }
   lastRhsFull_ = !useSparseWeno;
-  if (useSparseWeno && fused_) {
-    // linear pass (fast limiter test, KXRCF indicator, brick-boundary states)
-    // -> selection -> WENO and the limiter's exact sequence into rows ->
-    // fused reconstruction + Riemann + divergence + RK update
-    const bool lrn = learned_ && !forcePlain_;
+  // the learned selection does not read the KXRCF indicator; for the Euler
+  // equations it runs inside the linear pass, on the brick that pass stages
+  const bool lrn = useSparseWeno && learned_ && !forcePlain_ && hydro;
+  const bool fused = fusedNow();
+  const int cap = fused ? int(ncell_) : wsCap_;  // list positions with a row
+  const double *PW = sym_ && !pointOrder() ? parW_ : nullptr;
+  double *wi = lrn ? nullptr : WI_;
+  LearnArgs la;
+  if (lrn) {
+    la.eint = props_;
+    la.theta = thPrev;
+    la.nadFlag = nadFlag_;
+    la.P = netP_;
+    la.thr = netThr_;
+    la.wflag = wflag_;
+    la.list = list_;
+    la.counter = counter_;
+    la.pos = pos_;
+    la.cap = cap;
+  }
+  const double wThresh = cfg_.wenoThresh * std::pow(cfg_.dmin(), 1.5);
+  if (useSparseWeno && fused) {
+    // linear pass (fast limiter test, KXRCF indicator or the learned
+    // selection, brick-boundary states) -> selection -> WENO and the limiter's
+    // exact sequence into rows -> fused reconstruction + Riemann + divergence +
+    // RK update
     check(launch_zero(counter_ + 2, sizeof(int), stream_), "clear row count");
     timed("linear", [&] {
-      return launch_linear_surf(dim, nq, Uin, lrn ? nullptr : WI_, thNew, props_, grid_, faceWT_, ppList_,
-                                counter_ + 1, SB_, sb_, stream_);
+      return launch_linear_surf(dim, nq, Uin, wi, thNew, props_, grid_, parW_, ppList_, counter_ + 1, SB_, sb_,
+                                stream_, lrn ? &la : nullptr);
     });
-    if (lrn) {
+    if (!lrn)
       timed("select", [&] {
-        return launch_learned_select(dim, 5, Uin, props_, thPrev, nadFlag_, netP_, netThr_, wflag_, list_, counter_,
-                                     grid_, pos_, wsCap_, stream_);
-      });
-    } else {
-      const double wThresh = cfg_.wenoThresh * std::pow(cfg_.dmin(), 1.5);
-      timed("select", [&] {
-        return launch_select(dim, nq, Uin, WI_, thPrev, wflag_, list_, counter_, wThresh, grid_, pos_, wsCap_,
+        return launch_select(dim, nq, Uin, WI_, thPrev, wflag_, list_, counter_, wThresh, grid_, pos_, cap,
                              stream_);
       });
-    }
     timed("weno", [&] {
       return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_, counter_,
-                         FS_, wsCap_, stream_);
+                         FS_, cap, stream_);
     });
     timed("weno_post", [&] {
-      return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, FS_, wsCap_, stream_);
+      return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, FS_, cap, stream_);
     });
     timed("pp", [&] {
-      return launch_pp_rows(dim, nq, Uin, FS_, pos_, thNew, props_, wflag_, grid_, faceW_, ppList_, counter_ + 1,
+      return launch_pp_rows(dim, nq, Uin, FS_, pos_, thNew, props_, wflag_, grid_, parW_, ppList_, counter_ + 1,
                             counter_, counter_ + 2, stream_);
     });
     th_ ^= 1;
+    nPart_ = flux_rk_partials(dim, grid_, 0);
     timed("flux_rk", [&] {
-      return launch_flux_fused(dim, nq, Uin, faceWQ_, FS_, pos_, SB_, sb_, grid_, a, stream_);
+      return launch_flux_fused(dim, nq, Uin, parW_, FS_, pos_, SB_, sb_, grid_, a, stream_);
     });
     nRhsEval++;
     return;
   }
   if (useSparseWeno) {
-    // the learned selection does not read the KXRCF indicator; for the Euler
-    // equations it runs inside the linear pass, on the brick that pass stages
-    const bool lrn = learned_ && !forcePlain_ && hydro;
-    double *wi = lrn ? nullptr : WI_;
-    LearnArgs la;
-    if (lrn) {
-      la.eint = props_;
-      la.theta = thPrev;
-      la.nadFlag = nadFlag_;
-      la.P = netP_;
-      la.thr = netThr_;
-      la.wflag = wflag_;
-      la.list = list_;
-      la.counter = counter_;
-      la.pos = pos_;
-      la.cap = wsCap_;
-    }
     timed("linear", [&] {
       return launch_linear(dim, nq, nv_, Uin, FS_, wi, thNew, props_, grid_, faceW_, faceWT_, ppList_, counter_ + 1,
-                           stream_, lrn ? &la : nullptr);
+                           stream_, lrn ? &la : nullptr, PW);
     });
     if (hydro) {
-      if (!lrn) {
-        const double wThresh = cfg_.wenoThresh * std::pow(cfg_.dmin(), 1.5);
+      if (!lrn)
         timed("select", [&] {
-          return launch_select(dim, nq, Uin, WI_, thPrev, wflag_, list_, counter_, wThresh, grid_, pos_, wsCap_,
+          return launch_select(dim, nq, Uin, WI_, thPrev, wflag_, list_, counter_, wThresh, grid_, pos_, cap,
                                stream_);
         });
-      }
       timed("weno", [&] {
         return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_,
-                           counter_, WS_, wsCap_, stream_);
+                           counter_, WS_, cap, stream_);
       });
       timed("weno_post", [&] {
-        return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, WS_, wsCap_, stream_);
+        return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, WS_, cap, stream_);
       });
       timed("pp", [&] {
         return launch_pp_lanes(dim, nq, Uin, FS_, thNew, props_, wflag_, grid_, ppList_, counter_ + 1, stream_);
@@ -839,7 +825,13 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
     ar.pos = pos_;
     ar.ws = WS_;
   }
-  timed("flux_rk", [&] { return launch_flux_rk(dim, nq, nv_, Uin, FS_, grid_, ar, stream_, cfg_.fluxBrick); });
+  nPart_ = flux_rk_partials(dim, grid_, cfg_.fluxBrick);
+  // 3D Euler with WENO on every cell equals a learned run that picks every cell
+  if (pointOrder() || (hydro && dim == 3 && lastRhsFull_))
+    timed("flux_rk", [&] { return launch_flux_points(dim, nq, Uin, FS_, grid_, ar, stream_); });
+  else
+    timed("flux_rk",
+          [&] { return launch_flux_rk(dim, nq, nv_, Uin, FS_, grid_, ar, stream_, cfg_.fluxBrick); });
   nRhsEval++;
 }
 
@@ -862,7 +854,7 @@ double Solver::evalRHS(int which) {
   return readSpeed();
 }
 
-size_t Solver::carveEval(unsigned char *base, EvalBufs &b) const {
+size_t Solver::carveEval(unsigned char *base, EvalBufs &b, bool fuse) const {
   size_t off = 0;
   auto take = [&](size_t bytes) -> void * {
     off = (off + 255) / 256 * 256;
@@ -872,8 +864,9 @@ size_t Solver::carveEval(unsigned char *base, EvalBufs &b) const {
   };
   const size_t nc = size_t(ncell_), FQ = size_t(wts_.F) * wts_.Q, D = sizeof(double), I = sizeof(int);
   b.FS = static_cast<double *>(take(fs_elems(nc, int(FQ) * nv_) * D));
-  b.WS = WS_ ? static_cast<double *>(take(size_t(wsCap_) * FQ * nv_ * D)) : nullptr;
-  if (SB_) {
+  b.WS = nv_ == 5 && !fuse ? static_cast<double *>(take(size_t(wsCap_) * FQ * nv_ * D)) : nullptr;
+  b.SB = nullptr;
+  if (fuse) {
     Surf sb{};
     b.SB = static_cast<double *>(take(surf_elems(cfg_.dim, cfg_.nQuad, grid_, sb) * D));
   }
@@ -894,7 +887,10 @@ size_t Solver::carveEval(unsigned char *base, EvalBufs &b) const {
 
 size_t Solver::noAllocBytes() const {
   EvalBufs b;
-  return carveEval(nullptr, b);
+  // on thin grids the surface planes of the fused path take more than the
+  // staging of the unfused one (same results): a grid that either fits is taken
+  const size_t need = carveEval(nullptr, b, fusedNow());
+  return need > kNoAllocScratchBytes && fusedNow() ? carveEval(nullptr, b, false) : need;
 }
 
 double Solver::evalRhsNoAlloc(const double *U, double *rhs) {
@@ -904,7 +900,8 @@ double Solver::evalRhsNoAlloc(const double *U, double *rhs) {
                              std::to_string(kNoAllocScratchBytes) + " of the no-allocation entry point");
   unsigned char *base = static_cast<unsigned char *>(noalloc_scratch());
   EvalBufs b;
-  carveEval(base, b);
+  const bool fuse = fusedNow() && carveEval(nullptr, b, true) <= kNoAllocScratchBytes;
+  carveEval(base, b, fuse);
   // the solver's own buffers and evaluation state, put back on every exit
   struct Restore {
     Solver &s;
@@ -913,6 +910,7 @@ double Solver::evalRhsNoAlloc(const double *U, double *rhs) {
     bool sparse, lastFull, prof;
     int64_t nRhs;
     ~Restore() {
+      s.noFuse_ = false;
       s.FS_ = keep.FS;
       s.WS_ = keep.WS;
       s.SB_ = keep.SB;
@@ -942,6 +940,7 @@ double Solver::evalRhsNoAlloc(const double *U, double *rhs) {
             lastRhsFull_,
             profOn_,
             nRhsEval};
+  noFuse_ = !fuse;
   FS_ = b.FS;
   WS_ = b.WS;
   SB_ = b.SB;
@@ -1125,6 +1124,7 @@ void Solver::setIndicator(const float *params, int np, double threshold) {
   netThr_ = float(threshold);
   learned_ = true;
   forcePlain_ = false;
+  pathBuffers();
 }
 
 void Solver::collectSamples(float *X, float *Y, double tau) {
@@ -1154,7 +1154,7 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
   check(launch_zero(counter_, 2 * sizeof(int), stream_), "clear counters");
   check(launch_cell_props(dim, Uin, props_, grid_, stream_), "cell_props");
   check(launch_linear(dim, nq, nv_, Uin, FS_, WI_, thScratch, props_, grid_, faceW_, faceWT_, ppList_, counter_ + 1,
-                      stream_),
+                      stream_, nullptr, sym_ ? parW_ : nullptr),
         "linear");
   check(hipMemcpyAsync(FSlin_, FS_, fsBytes, hipMemcpyDeviceToDevice, stream_), "copy linear states");
   check(launch_weno(dim, nq, nv_, Uin, FS_, thScratch, grid_, faceW_, derivW_, faceWC_, derivWS_, nullptr, nullptr,
@@ -1345,13 +1345,13 @@ void Solver::uploadWeights() {
                          nCell ? wts_.cell.data() : nullptr);
     check(hipMemcpy(faceWC_, wc.data(), wc.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
   }
-  if (faceWQ_) {  // full-stencil face weights per point: [Q][C][F]
-    const int Q = wts_.Q, F = wts_.F;
-    std::vector<double> wq(size_t(Q) * C * F);
-    for (int q = 0; q < Q; q++)
-      for (int n = 0; n < C; n++)
-        for (int f = 0; f < F; f++) wq[(size_t(q) * C + n) * F + f] = wts_.face[size_t(f * Q + q) * C + n];
-    check(hipMemcpy(faceWQ_, wq.data(), wq.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
+  if (parW_) {  // parity coefficients of the full-stencil face weights, [type][C]
+    std::vector<double> pw;
+    sym_ = wts_.dim == 3 ? parity_face_list<3>(wts_.nq, wts_.face.data(), pw)
+                         : parity_face_list<2>(wts_.nq, wts_.face.data(), pw);
+    if (sym_) check(hipMemcpy(parW_, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
+    fused_ = fusedWanted_ && sym_;
+    pathBuffers();
   }
   if (cellW_) {
     const int NI = wts_.nqCell;
@@ -1373,6 +1373,16 @@ void Solver::uploadWeights() {
         for (int q = 0; q < PI; q++) wi[(size_t(ps) * C + n) * PI + q] = wts_.cell[size_t(ps * PI + q) * C + n];
     check(hipMemcpy(mhdWT_, mw.data(), mw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
   }
+}
+// Buffers of the sparse-mode path in use (Euler): the fused one keeps the
+// brick-boundary planes and a row per listed cell (in FS_), the unfused one a
+// compact WENO staging for up to a quarter of the cells.
+void Solver::pathBuffers() {
+  if (nv_ != 5) return;
+  const size_t nc = size_t(ncell_), FQ = size_t(wts_.F) * wts_.Q;
+  wsCap_ = int(std::max<size_t>(1, (nc + 3) / 4));
+  if (fusedNow() && !SB_) SB_ = dalloc<double>(surf_elems(cfg_.dim, cfg_.nQuad, grid_, sb_), "surface planes");
+  if (!fusedNow() && !WS_) WS_ = dalloc<double>(size_t(wsCap_) * FQ * nv_, "compact WENO states");
 }
 void Solver::sync() const { check(hipStreamSynchronize(stream_), "sync"); }
 

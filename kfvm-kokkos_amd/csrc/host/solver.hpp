@@ -116,7 +116,8 @@ class Solver {
   };
   // Lay the buffers of this solver's evaluation out from base (256-byte
   // aligned; base null: sizes only) and return the bytes they span.
-  size_t carveEval(unsigned char *base, EvalBufs &b) const;
+  // fuse: those of the fused path.
+  size_t carveEval(unsigned char *base, EvalBufs &b, bool fuse) const;
   struct Prof {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
     double ms = 0.0;
@@ -131,6 +132,12 @@ class Solver {
   void pipeline(const double *Uin, const RKArgs &a);
   void pipelineMhd(const double *Uin, const RKArgs &a);
   void uploadWeights();
+  void pathBuffers();
+  // 3D Euler with the learned selection keeps one order of operations
+  // (points5.hpp): its choice of cells reads the rounding of the state
+  bool pointOrder() const { return learned_ && nv_ == 5 && cfg_.dim == 3; }
+  bool fusedNow() const { return fused_ && !noFuse_ && !pointOrder(); }
+  bool noFuse_ = false;  // this evaluation's scratch only fits the unfused path
   double readSpeed();
   bool nadFails();
   int takeStepSlices();
@@ -152,10 +159,11 @@ class Solver {
   int *pos_ = nullptr;    // per cell: its row in WS_ (fused path: in FS_), or -1
   int wsCap_ = 0;
   // Euler sparse mode, fused path: the brick-boundary face states of the linear
-  // pass (surface planes) and the face weights per point [Q][C][F]; listed
-  // cells keep their states in rows of FS_
-  bool fused_ = false;
-  double *SB_ = nullptr, *faceWQ_ = nullptr;
+  // pass (surface planes); listed cells keep their states in rows of FS_.
+  // sym_: the full-stencil weights are mirror-symmetric, parW_ their parity
+  // coefficients [type][C]
+  bool fused_ = false, fusedWanted_ = false, sym_ = false;
+  double *SB_ = nullptr, *parW_ = nullptr;
   Surf sb_{};
   double *props_ = nullptr;  // per-cell internal energy and sound speed [2][ncell]
   double *theta_[2] = {nullptr, nullptr};  // positivity theta: previous RHS / this RHS
