@@ -126,7 +126,7 @@ hipError_t launch_flow_stats(int dim, int nv, const double *U, const Grid &g, do
 }
 hipError_t launch_mhd_chmax(int dim, const double *spd, const Grid &g, unsigned long long *chBits, hipStream_t s) {
   (void)dim;
-  const unsigned nb = std::min<unsigned>(stage_blocks(g.ncell), 2048u);
+  const unsigned nb = std::min<unsigned>(stage_blocks(g.ncell), 256u);
   hipLaunchKernelGGL(dev::k_mhd_chmax, dim3(nb), dim3(dev::BLK), 0, s, spd, int64_t(g.ncell), chBits);
   return hipGetLastError();
 }

@@ -51,7 +51,8 @@ template <int D, int NQ>
 hipError_t Launch<D, NQ>::select(const double *U, const double *WI, const double *theta, double *wflag,
                                  int *list, int *counter, double wThresh, const Grid &g, int *pos, int cap,
                                  hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_select<D, NQ>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, WI, theta, wflag,
+  constexpr int nt = dev::SelectBlock<D, NQ>::NT;
+  hipLaunchKernelGGL((dev::k_select<D, NQ>), dim3((unsigned(g.ncell) + nt - 1) / nt), dim3(nt), 0, s, U, WI, theta, wflag,
                      list, counter, wThresh, g, pos, cap);
   return hipGetLastError();
 }
@@ -181,7 +182,8 @@ hipError_t LaunchMhd<D, NQ>::linear(const double *U, double *FS, double *SRC, do
 template <int D, int NQ>
 hipError_t LaunchMhd<D, NQ>::select(const double *U, const double *WI, const double *theta, double *wflag,
                                      int *list, int *counter, double wThresh, const Grid &g, hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_select<D, NQ, dev::Mhd>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, WI,
+  constexpr int nt = dev::SelectBlock<D, NQ>::NT;
+  hipLaunchKernelGGL((dev::k_select<D, NQ, dev::Mhd>), dim3((unsigned(g.ncell) + nt - 1) / nt), dim3(nt), 0, s, U, WI,
                      theta, wflag, list, counter, wThresh, g, nullptr, 0);
   return hipGetLastError();
 }

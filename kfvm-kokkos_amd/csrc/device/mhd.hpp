@@ -821,10 +821,21 @@ __global__ __launch_bounds__(BLK) void k_mhd_chmax(const double *__restrict__ sp
                                                    unsigned long long *__restrict__ chBits) {
   __shared__ double sh[BLK];
   double lam = 0.0, vel = 0.0;
-  for (int64_t c = int64_t(blockIdx.x) * BLK + threadIdx.x; c < ncell; c += int64_t(gridDim.x) * BLK) {
-    const double l = spd[c], v = spd[ncell + c];
-    lam = l > lam ? l : lam;
-    vel = v > vel ? v : vel;
+  // few workgroups (two atomics each), eight cells of a thread in flight
+  const int64_t stride = int64_t(gridDim.x) * BLK;
+  for (int64_t c0 = int64_t(blockIdx.x) * BLK + threadIdx.x; c0 < ncell; c0 += 8 * stride) {
+    double l[8], v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const int64_t c = c0 + e * stride;
+      l[e] = c < ncell ? spd[c] : 0.0;
+      v[e] = c < ncell ? spd[ncell + c] : 0.0;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      lam = l[e] > lam ? l[e] : lam;
+      vel = v[e] > vel ? v[e] : vel;
+    }
   }
   const double bl = block_max(lam, sh, threadIdx.x);
   const double bv = block_max(vel, sh, threadIdx.x);

@@ -307,47 +307,81 @@ __device__ inline void list_append(bool live, bool flagged, int c, int *__restri
   if (pos && live) pos[c] = idx >= 0 && idx < cap ? idx : -1;
 }
 
+// The same with one atomic per workgroup of NW waves (every thread calls it).
+// Atomics on the one counter are served one after another, about 10 ns each:
+// with one per wave they were most of the selector's time.
+template <int NW>
+__device__ inline void list_append_block(bool live, bool flagged, int c, int *__restrict__ list,
+                                         int *__restrict__ counter, int *__restrict__ pos, int cap) {
+  __shared__ int cnt[NW + 1];
+  const unsigned long long mask = __ballot(flagged);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) cnt[wave] = __popcll(mask);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int sum = 0;
+    for (int w = 0; w < NW; w++) {
+      const int n = cnt[w];
+      cnt[w] = sum;
+      sum += n;
+    }
+    cnt[NW] = sum ? atomicAdd(counter, sum) : 0;
+  }
+  __syncthreads();
+  int idx = -1;
+  if (flagged) {
+    idx = cnt[NW] + cnt[wave] + __popcll(mask & ((1ull << lane) - 1ull));
+    list[idx] = c;
+  }
+  if (pos && live) pos[c] = idx >= 0 && idx < cap ? idx : -1;
+}
+
 // ------------------------------------------------------------ KXRCF selector
+// Threads per workgroup: as many as the 2 F Q loaded values leave registers for.
+template <int D, int NQ>
+struct SelectBlock {
+  static constexpr int NT = D == 3 && NQ == 3 ? 512 : 1024;
+};
+
 template <int D, int NQ, class P = Hydro>
-__global__ __launch_bounds__(BLK) void k_select(const double *__restrict__ U,
+__global__ __launch_bounds__((SelectBlock<D, NQ>::NT)) void k_select(const double *__restrict__ U,
                                                 const double *__restrict__ WI,
                                                 const double *__restrict__ theta,
                                                 double *__restrict__ wflag, int *__restrict__ list,
                                                 int *__restrict__ counter, double wThresh,
                                                 Grid g, int *__restrict__ pos, int cap) {
   constexpr int F = Shape<D, NQ>::F, Q = Shape<D, NQ>::Q;
-  const int c = blockIdx.x * BLK + threadIdx.x;
+  const int c = blockIdx.x * SelectBlock<D, NQ>::NT + threadIdx.x;
   bool flagged = false;
   if (c < g.ncell) {
     int i, j, k;
     cell_ijk<D>(c, g, i, j, k);
     const size_t nc = g.ncell;
-    double maxJump = 0.0;
+    // The neighbour's opposite face, or the cell's own face beyond a wall (no
+    // jump): every load is unconditional, so all 2 F Q of a cell are in flight
+    // at once (with a branch per face they waited for one another).
+    const double *const own = WI + fs_base(c, F * Q);
+    double win[F * Q], wout[F * Q];
 #pragma unroll
     for (int f = 0; f < F; f++) {
       const int ax = f >> 1, hi = f & 1;
-      int ni = i, nj = j, nk = k;
-      if (ax == 0) ni += hi ? 1 : -1;
-      if (ax == 1) nj += hi ? 1 : -1;
-      if (ax == 2) nk += hi ? 1 : -1;
       const int n_ax = ax == 0 ? g.nx : (ax == 1 ? g.ny : g.nz);
-      const int pos = ax == 0 ? ni : (ax == 1 ? nj : nk);
-      bool inside = pos >= 0 && pos < n_ax;
-      if (!inside && g.bc[f] == 0) {
-        inside = true;
-        if (ax == 0) ni = (ni + g.nx) % g.nx;
-        if (ax == 1) nj = (nj + g.ny) % g.ny;
-        if (ax == 2) nk = (nk + g.nz) % g.nz;
-      }
-      const size_t cn = (size_t(nk) * g.ny + nj) * g.nx + ni;
-      const int fo = f ^ 1;  // opposite face of the neighbour
+      const int stride = ax == 0 ? 1 : (ax == 1 ? g.nx : g.nx * g.ny);
+      const int at = ax == 0 ? i : (ax == 1 ? j : k);
+      const bool edge = hi ? at == n_ax - 1 : at == 0;
+      const int step = (hi ? 1 : -1) - (edge ? (hi ? n_ax : -n_ax) : 0);  // across a periodic edge: wraps
+      const bool wall = edge && g.bc[f] != 0;
+      const double *other = WI + fs_base(size_t(c + (wall ? 0 : step * stride)), F * Q);
+      const int fo = wall ? f : (f ^ 1);
 #pragma unroll
       for (int q = 0; q < Q; q++) {
-        const double win = WI[fs_base(c, F * Q) + size_t(f * Q + q) * FSB];
-        const double wout = inside ? WI[fs_base(cn, F * Q) + size_t(fo * Q + q) * FSB] : win;
-        maxJump = fmax(maxJump, fabs(wout - win));
+        win[f * Q + q] = own[size_t(f * Q + q) * FSB];
+        wout[f * Q + q] = other[size_t(fo * Q + q) * FSB];
       }
     }
+    double maxJump = 0.0;
+#pragma unroll
+    for (int p = 0; p < F * Q; p++) maxJump = fmax(maxJump, fabs(wout[p] - win[p]));
     double uc[P::NV];
 #pragma unroll
     for (int v = 0; v < P::NV; v++) uc[v] = U[size_t(v) * nc + c];
@@ -355,7 +389,7 @@ __global__ __launch_bounds__(BLK) void k_select(const double *__restrict__ U,
     flagged = ind >= wThresh || theta[c] < 1.0;
     wflag[c] = flagged ? 1.0 : 0.0;
   }
-  list_append(c < g.ncell, flagged, c, list, counter, pos, cap);
+  list_append_block<SelectBlock<D, NQ>::NT / 64>(c < g.ncell, flagged, c, list, counter, pos, cap);
 }
 
 // ---------------------------------------------------------------- KFVM-WENO
