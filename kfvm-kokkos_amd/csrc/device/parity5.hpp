@@ -107,9 +107,13 @@ __device__ __forceinline__ void parity_points(const double (&t)[SInfo<D>::C], WP
   });
 }
 
-// Stencil values of a brick cell from one staged plane (p: its box corner).
+// Stencil values of a brick cell from one staged plane (corner: its box corner).
+// The offset is opaque at each call: the planes do not change, so the compiler
+// would otherwise keep one sweep's values for the next and spill them.
 template <int D, class Bx>
-__device__ __forceinline__ void load_stencil(const double *p, double (&t)[SInfo<D>::C]) {
+__device__ __forceinline__ void load_stencil(const double *plane, int corner, double (&t)[SInfo<D>::C]) {
+  asm volatile("" : "+v"(corner));
+  const double *p = plane + corner;
   static_for<SInfo<D>::C>([&](auto nn) KFVM_INLINE {
     constexpr int n = decltype(nn)::value;
     constexpr int o = (StTab<D>::ST.off[n][0] + Bx::H) + Bx::LX * (StTab<D>::ST.off[n][1] + Bx::H) +
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(RBox<D>::NT, D == 3 && NQ == 3 ? 2 : 3) void k_line
       static_for<5>([&](auto vv) KFVM_INLINE {
         constexpr int v = decltype(vv)::value;
         double t[C];
-        load_stencil<D, Bx>(lds + v * NP + corner, t);
+        load_stencil<D, Bx>(lds + v * NP, corner, t);
         parity_transform<D>(t);
         // opaque per variable, so that the coefficients stay scalar loads next
         // to their products instead of being hoisted out of the loop
@@ -256,7 +260,7 @@ __global__ __launch_bounds__(RBox<D>::NT, D == 3 && NQ == 3 ? 2 : 3) void k_line
         for (int p0 = 0; p0 < NPT; p0 += IT) {
 #pragma unroll
           for (int p = 0; p < IT; p++) {
-            wi[size_t(p0 + p) * FSB] = (gm1 * msq[p]) / pow(rho[p], g.gamma);
+            wi[size_t(p0 + p) * FSB] = (gm1 * msq[p]) * pow_pos(rho[p], -g.gamma);
             __builtin_amdgcn_sched_barrier(0);
           }
 #pragma unroll
@@ -514,7 +518,7 @@ __global__ __launch_bounds__(RBox<D>::NT, 2) void k_flux_par(const double *__res
 #pragma unroll
       for (int w = 0; w < 5; w++) {
         double t[C];
-        load_stencil<D, Bx>(lds + rv[w] * NP + corner, t);
+        load_stencil<D, Bx>(lds + rv[w] * NP, corner, t);
         parity_transform<D>(t);
         parity_points<D, NQ, A>(t, (const cdouble *)w0, pt[w]);
         __builtin_amdgcn_sched_barrier(0);  // one variable's stencil in registers at a time

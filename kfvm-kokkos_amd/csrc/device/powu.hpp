@@ -79,6 +79,7 @@ KFVM_POWU_HD inline double powu(double x, double y) {
 #ifdef __HIPCC__
 namespace dev {
 __device__ inline double div_n(double a, double b);  // physics.hpp
+__device__ inline double rcp_n(double x);
 }
 #endif
 
@@ -100,6 +101,74 @@ KFVM_POWU_HD inline double pow_ratio(double a, double b, double y) {
 #else
   return exp_y_ln((m - n) / (m + n), e, y);
 #endif
+}
+
+// x^y for |y| <= 2^10 (an adiabatic exponent).  ln |x| as a head and a tail:
+// |x| = m 2^e, m in [1/sqrt 2, sqrt 2), s = (m-1)/(m+1) with its remainder,
+// 2 atanh(s) by Taylor to s^23; the product with y keeps its rounding error,
+// which enters exp's reduced argument.  Within one ulp of powl
+// (tests/test_pow_pos.py), the bound of the library's pow, of whose 190
+// instructions it takes about 80.
+KFVM_POWU_HD inline double pow_pos(double x, double y) {
+  const double ax = std::fabs(x);
+  constexpr double LN2_HEAD = 0.6931467056274414;
+  constexpr double LN2_TAIL = 4.7493250390316726e-07;
+  constexpr double INV_LN2 = 1.4426950408889634;
+  int e;
+  double m = std::frexp(ax, &e);
+  if (m < 0.70710678118654752) {
+    m *= 2.0;
+    e -= 1;
+  }
+  const double f = m - 1.0, d = m + 1.0, dl = m - (d - 1.0);
+#ifdef __HIP_DEVICE_COMPILE__
+  const double r = dev::rcp_n(d);
+#else
+  const double r = 1.0 / d;
+#endif
+  const double s = f * r, sl = std::fma(-s, dl, std::fma(-s, d, f)) * r;
+  const double z = s * s;
+  double p = 1.0 / 23.0;
+  p = std::fma(p, z, 1.0 / 21.0);
+  p = std::fma(p, z, 1.0 / 19.0);
+  p = std::fma(p, z, 1.0 / 17.0);
+  p = std::fma(p, z, 1.0 / 15.0);
+  p = std::fma(p, z, 1.0 / 13.0);
+  p = std::fma(p, z, 1.0 / 11.0);
+  p = std::fma(p, z, 1.0 / 9.0);
+  p = std::fma(p, z, 1.0 / 7.0);
+  p = std::fma(p, z, 1.0 / 5.0);
+  p = std::fma(p, z, 1.0 / 3.0);
+  // ln x = th + tl: e ln2_head (exact) + 2 s, then the small terms
+  const double de = double(e), a = de * LN2_HEAD, b = 2.0 * s;
+  const double sum = a + b, bb = sum - a;
+  const double low = (a - (sum - bb)) + (b - bb) + std::fma(de, LN2_TAIL, 2.0 * std::fma(s * z, p, sl));
+  const double th = sum + low, tl = low - (th - sum);
+  const double t = y * th, u = std::fma(y, th, -t) + y * tl;
+  const double n = std::rint(t * INV_LN2);
+  const double w = std::fma(-n, LN2_HEAD, t) + (u - n * LN2_TAIL);
+  double q = 1.6059043836821613e-10;  // 1/13!
+  q = std::fma(q, w, 2.08767569878681e-09);
+  q = std::fma(q, w, 2.505210838544172e-08);
+  q = std::fma(q, w, 2.755731922398589e-07);
+  q = std::fma(q, w, 2.7557319223985893e-06);
+  q = std::fma(q, w, 2.48015873015873e-05);
+  q = std::fma(q, w, 0.0001984126984126984);
+  q = std::fma(q, w, 0.001388888888888889);
+  q = std::fma(q, w, 0.008333333333333333);
+  q = std::fma(q, w, 0.041666666666666664);
+  q = std::fma(q, w, 0.16666666666666666);
+  q = std::fma(q, w, 0.5);
+  const double c = std::fma(q * w, w, w);  // e^w - 1
+  double v = std::ldexp(1.0 + c, int(n));
+  // zero, infinity, and a negative base (real for whole y only)
+  const double inf = __builtin_inf();
+  if (ax == 0.0 || ax == inf) v = y == 0.0 ? 1.0 : ((y > 0.0) == (ax == 0.0) ? 0.0 : inf);
+  if (x < 0.0) {
+    const double h = 0.5 * y;
+    v = y != std::rint(y) ? __builtin_nan("") : (h != std::rint(h) ? -v : v);
+  }
+  return v;
 }
 
 }  // namespace kfvm
