@@ -129,8 +129,9 @@ struct RKArgs {
 };
 
 // Euler: per-cell internal energy and sound speed, props [2][ncell], read by
-// the limiter bounds of launch_linear and launch_weno_post.
-hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s);
+// the limiter bounds of launch_linear and launch_weno_post.  Also clears the
+// four list counters of the evaluation.
+hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid &g, int *counter, hipStream_t s);
 // Linear reconstruction, KXRCF indicator and positivity limiter (all cells).
 // W0: full-stencil face weights [F*Q][C]; W0T: the same regrouped per pass
 // of linear_pass_points(dim, nq) points as [F*Q/P][C][P].  Euler: cells
@@ -206,11 +207,13 @@ hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double
                             double *WS, int cap, hipStream_t s);
 // GLM-MHD (9 variables).  SRC [(p * 9 + v)][ncell]: states, then source
 // terms, at the NQ^D interior points; props [2][ncell]: per-cell internal
-// energy and sound speed (launch_mhd_props, before the linear pass or WENO);
+// energy and sound speed (launch_mhd_props, before the linear pass or WENO,
+// which also clears the list counters and chBits);
 // spd [2][ncell]: per-cell maxima of c_f + |u| and |u| over the cell's limited
 // face states, which launch_mhd_chmax folds into chBits for the flux kernel's
 // cleaning speed.
-hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s);
+hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid &g, int *counter,
+                            unsigned long long *chBits, hipStream_t s);
 // WT: full-stencil weights per pass, the face passes [F*Q/P][C][P]
 // (P = linear_pass_points) then the interior passes [NQ^D/PI][C][PI]
 // (PI = mhd_interior_pass_points).  Cells whose states violate a limiter
@@ -264,9 +267,12 @@ hipError_t launch_stage_pre_slices(int nv, const double *Uprev, const double *K,
                                    double *Utmp, const double *sliceDt, double beta, double bhat, int ncell,
                                    int cellsPerSlice, hipStream_t s);
 hipError_t launch_stage_pre(int nv, const double *Uprev, const double *K, double *U, double *Uhat,
-                            double *Utmp, double betaDt, double bhatDt, int ncell, hipStream_t s);
+                            double *Utmp, double betaDt, double bhatDt, int ncell, unsigned long long *vmax,
+                            hipStream_t s);  // vmax (may be null): cleared
+// out[4], host memory the device can write: error sum, positivity minimum, the
+// bits of *vmax and, in the bits of out[3], *counter
 hipError_t launch_finalize(const double *errPartial, const double *posPartial, int nPart,
-                           double *out, hipStream_t s);
+                           const unsigned long long *vmax, const int *counter, double *out, hipStream_t s);
 hipError_t launch_fill(double *p, double v, size_t n, hipStream_t s);
 // Zero `bytes` (a multiple of 4) with a kernel, not a memset (graph capture).
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);

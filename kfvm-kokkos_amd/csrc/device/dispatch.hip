@@ -16,8 +16,8 @@ namespace kfvm {
   } while (0)
 #define KFVM_SELECT(dim, nq, CALL) KFVM_SELECT_OF(Launch, dim, nq, CALL)
 
-hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s) {
-  KFVM_SELECT(dim, 2, L::cell_props(U, props, g, s));
+hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid &g, int *counter, hipStream_t s) {
+  KFVM_SELECT(dim, 2, L::cell_props(U, props, g, counter, s));
 }
 
 hipError_t launch_linear(int dim, int nq, int nv, const double *U, double *FS, double *WI,
@@ -95,8 +95,9 @@ hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double
   KFVM_SELECT(dim, nq, L::weno_post(U, FS, thetaNew, props, g, list, counter, WS, cap, s));
 }
 
-hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid &g, hipStream_t s) {
-  KFVM_SELECT_OF(LaunchMhd, dim, 2, L::props(U, props, g, s));
+hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid &g, int *counter,
+                            unsigned long long *chBits, hipStream_t s) {
+  KFVM_SELECT_OF(LaunchMhd, dim, 2, L::props(U, props, g, counter, chBits, s));
 }
 hipError_t launch_mhd_linear(int dim, int nq, const double *U, double *FS, double *SRC, double *WI,
                              double *thetaNew, double *spd, const double *props, const Grid &g, const double *WT,
@@ -150,16 +151,17 @@ int flux_rk_partials(int dim, const Grid &g, int shape) {
 }
 
 hipError_t launch_stage_pre(int nv, const double *Uprev, const double *K, double *U, double *Uhat,
-                            double *Utmp, double betaDt, double bhatDt, int ncell, hipStream_t s) {
+                            double *Utmp, double betaDt, double bhatDt, int ncell, unsigned long long *vmax,
+                            hipStream_t s) {
   if (nv == 5)
     hipLaunchKernelGGL((dev::k_stage_pre<5>), dim3(stage_blocks(ncell)), dim3(dev::BLK), 0, s, Uprev,
-                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell);
+                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell, vmax);
   else if (nv == 1)
     hipLaunchKernelGGL((dev::k_stage_pre<1>), dim3(stage_blocks(ncell)), dim3(dev::BLK), 0, s, Uprev,
-                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell);
+                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell, vmax);
   else if (nv == 9)
     hipLaunchKernelGGL((dev::k_stage_pre<9>), dim3(stage_blocks(ncell)), dim3(dev::BLK), 0, s, Uprev,
-                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell);
+                       K, U, Uhat, Utmp, betaDt, bhatDt, ncell, vmax);
   else
     return hipErrorInvalidValue;
   return hipGetLastError();
@@ -194,8 +196,8 @@ hipError_t launch_finalize_slices(const double *errPartial, const double *posPar
 }
 
 hipError_t launch_finalize(const double *errPartial, const double *posPartial, int nPart,
-                           double *out, hipStream_t s) {
-  hipLaunchKernelGGL(dev::k_finalize, dim3(1), dim3(1024), 0, s, errPartial, posPartial, nPart, out);
+                           const unsigned long long *vmax, const int *counter, double *out, hipStream_t s) {
+  hipLaunchKernelGGL(dev::k_finalize, dim3(1), dim3(1024), 0, s, errPartial, posPartial, nPart, vmax, counter, out);
   return hipGetLastError();
 }
 

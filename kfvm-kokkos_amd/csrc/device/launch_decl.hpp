@@ -16,7 +16,7 @@ namespace kfvm {
 template <int D, int NQ>
 struct Launch {
   static unsigned bricks(const Grid &g);
-  static hipError_t cell_props(const double *U, double *props, const Grid &g, hipStream_t s);
+  static hipError_t cell_props(const double *U, double *props, const Grid &g, int *counter, hipStream_t s);
   static hipError_t linear(int nv, const double *U, double *FS, double *WI, double *thetaNew,
                            const double *props, const Grid &g, const double *W0, const double *W0T,
                            int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la, const double *PW);
@@ -67,7 +67,8 @@ struct Launch {
 template <int D, int NQ>
 struct LaunchMhd {
   static unsigned bricks(const Grid &g);
-  static hipError_t props(const double *U, double *props, const Grid &g, hipStream_t s);
+  static hipError_t props(const double *U, double *props, const Grid &g, int *counter, unsigned long long *chBits,
+                          hipStream_t s);
   static hipError_t linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew, double *spd,
                                const double *props, const Grid &g, const double *WT, int *ppList, int *ppCount,
                                hipStream_t s);

@@ -19,8 +19,9 @@ unsigned Launch<D, NQ>::bricks(const Grid &g) {
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::cell_props(const double *U, double *props, const Grid &g, hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_cell_props<D>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, props, g);
+hipError_t Launch<D, NQ>::cell_props(const double *U, double *props, const Grid &g, int *counter, hipStream_t s) {
+  hipLaunchKernelGGL((dev::k_cell_props<D>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, props, g,
+                     counter);
   return hipGetLastError();
 }
 
@@ -164,8 +165,10 @@ unsigned LaunchMhd<D, NQ>::bricks(const Grid &g) {
 }
 
 template <int D, int NQ>
-hipError_t LaunchMhd<D, NQ>::props(const double *U, double *props, const Grid &g, hipStream_t s) {
-  hipLaunchKernelGGL((dev::k_mhd_props<D>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, props, g);
+hipError_t LaunchMhd<D, NQ>::props(const double *U, double *props, const Grid &g, int *counter,
+                                   unsigned long long *chBits, hipStream_t s) {
+  hipLaunchKernelGGL((dev::k_mhd_props<D>), dim3(stage_blocks(g.ncell)), dim3(dev::BLK), 0, s, U, props, g,
+                     counter, chBits);
   return hipGetLastError();
 }
 

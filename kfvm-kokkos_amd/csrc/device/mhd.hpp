@@ -432,8 +432,12 @@ __device__ inline void mhd_scale(double *__restrict__ FS, double *__restrict__ S
 // momenta and the field, so mirrored wall cells need no sign.
 template <int D>
 __global__ __launch_bounds__(BLK) void k_mhd_props(const double *__restrict__ U, double *__restrict__ props,
-                                                   Grid g) {
+                                                   Grid g, int *__restrict__ counter,
+                                                   unsigned long long *__restrict__ chBits) {
   const int c = blockIdx.x * BLK + threadIdx.x;
+  // the evaluation's list counters and cleaning-speed maxima: it is its first kernel
+  if (c < 4) counter[c] = 0;
+  if (c < 2) chBits[c] = 0ull;
   if (c >= g.ncell) return;
   const size_t nc = g.ncell;
   double s[9];

@@ -295,8 +295,10 @@ __global__ __launch_bounds__(RBox<D>::NT, 3) void k_linear_fused(
 
 template <int D>
 __global__ __launch_bounds__(BLK) void k_cell_props(const double *__restrict__ U,
-                                                    double *__restrict__ props, Grid g) {
+                                                    double *__restrict__ props, Grid g,
+                                                    int *__restrict__ counter) {
   const int c = blockIdx.x * BLK + threadIdx.x;
+  if (c < 4) counter[c] = 0;  // the evaluation's list counters: it is its first kernel
   if (c >= g.ncell) return;
   const size_t nc = g.ncell;
   double s[5];

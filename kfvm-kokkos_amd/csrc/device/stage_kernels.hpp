@@ -1086,8 +1086,10 @@ __global__ __launch_bounds__(BLK) void k_stage_pre(const double *__restrict__ Up
                                                    const double *__restrict__ K,
                                                    double *__restrict__ U, double *__restrict__ Uhat,
                                                    double *__restrict__ Utmp, double betaDt,
-                                                   double bhatDt, int ncell) {
+                                                   double bhatDt, int ncell,
+                                                   unsigned long long *__restrict__ vmax) {
   const int c = blockIdx.x * BLK + threadIdx.x;
+  if (c == 0 && vmax) *vmax = 0ull;  // the step's running maximum
   if (c >= ncell) return;
 #pragma unroll
   for (int v = 0; v < NV; v++) {
@@ -1159,10 +1161,13 @@ __global__ __launch_bounds__(BLK) void k_finalize_slices(const double *__restric
   }
 }
 
-// Deterministic final reduction of the per-block partials.
+// Deterministic final reduction of the per-block partials.  out is host memory:
+// the host reads [error sum, positivity minimum, speed bits, WENO count] after
+// the stream, without a copy per value.
 __global__ __launch_bounds__(1024) void k_finalize(const double *__restrict__ errPartial,
                                                    const double *__restrict__ posPartial,
-                                                   int nPart, double *__restrict__ out) {
+                                                   int nPart, const unsigned long long *__restrict__ vmax,
+                                                   const int *__restrict__ counter, double *__restrict__ out) {
   __shared__ double se[1024], sp[1024];
   double e = 0.0, p = 1.0;
   for (int t = threadIdx.x; t < nPart; t += 1024) {
@@ -1184,6 +1189,8 @@ __global__ __launch_bounds__(1024) void k_finalize(const double *__restrict__ er
   if (threadIdx.x == 0) {
     out[0] = se[0];
     out[1] = sp[0];
+    out[2] = __longlong_as_double((long long)*vmax);
+    out[3] = __longlong_as_double((long long)*counter);
   }
 }
 

@@ -189,7 +189,6 @@ void Solver::setup() {
   const int nPartMax = std::max(nPart_, flux_rk_partials(cfg_.dim, grid_, 0));
   errPart_ = dalloc<double>(size_t(nPartMax), "err partials");
   posPart_ = dalloc<double>(size_t(nPartMax), "pos partials");
-  redOut_ = dalloc<double>(2, "reduction");
   vmax_ = dalloc<unsigned long long>(size_t(slices_), "vmax");
   if (slices_ > 1) {
     sDtDev_ = dalloc<double>(size_t(slices_), "slice dt");
@@ -219,7 +218,7 @@ void Solver::setup() {
   check(launch_fill(theta_[0], 1.0, nc, stream_), "fill theta");
   check(launch_fill(theta_[1], 1.0, nc, stream_), "fill theta");
   check(launch_fill(wflag_, 0.0, nc, stream_), "fill wflag");
-  check(launch_zero(counter_, sizeof(int), stream_), "clear counter");
+  check(launch_zero(counter_, 4 * sizeof(int), stream_), "clear counter");
 
   const bool restart = !cfg_.restartFile.empty();
   if (cfg_.plotFreq > 0.0 || cfg_.ckptFreq > 0 || restart) writer_.reset(new Writer(cfg_));
@@ -594,7 +593,7 @@ void Solver::release() noexcept {
   } catch (...) {
   }
   void *bufs[] = {SRC_, cellW_, cellWS_, diffM_, chBits_, U_[0], U_[1], Uprev_, Uhat_, K_, Utmp_, FS_, WI_, props_, theta_[0], theta_[1], wflag_, list_, counter_, ppList_,
-                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, redOut_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
+                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
   if (stream_) (void)hipStreamSynchronize(stream_);
   for (auto &kv : graphs_)
     if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
@@ -669,8 +668,8 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
   double *thNew = theta_[th_ ^ 1];
   lastRhsFull_ = !useSparseWeno;
   // counter_: [0] WENO cells, [1] cells of the linear pass for the limiter's exact sequence
-  check(launch_zero(counter_, 2 * sizeof(int), stream_), "clear counters");
-  timed("cell_props", [&] { return launch_mhd_props(dim, Uin, props_, grid_, stream_); });
+  // (cleared, like chBits_, by the first kernel)
+  timed("cell_props", [&] { return launch_mhd_props(dim, Uin, props_, grid_, counter_, chBits_, stream_); });
   if (useSparseWeno) {
     const bool lrn = learned_ && !forcePlain_;
     timed("linear", [&] {
@@ -704,7 +703,6 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
     useSparseWeno = cfg_.wenoThresh > 0.0;
   }
   th_ ^= 1;
-  check(launch_zero(chBits_, 2 * sizeof(unsigned long long), stream_), "clear speeds");
   timed("chmax", [&] { return launch_mhd_chmax(dim, spd_, grid_, chBits_, stream_); });
   RKArgs a = a0;
   a.chBits = chBits_;
@@ -725,10 +723,8 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   double *thNew = theta_[th_ ^ 1];
   // counter_: [0] WENO cells, [1] cells of the linear pass for the limiter's
   // exact sequence (ppList_)
-  if (hydro) {
-    check(launch_zero(counter_, 2 * sizeof(int), stream_), "clear counters");
-    timed("cell_props", [&] { return launch_cell_props(dim, Uin, props_, grid_, stream_); });
-  }
+  if (hydro)  // clears the counters
+    timed("cell_props", [&] { return launch_cell_props(dim, Uin, props_, grid_, counter_, stream_); });
   lastRhsFull_ = !useSparseWeno;
   // the learned selection does not read the KXRCF indicator; for the Euler
   // equations it runs inside the linear pass, on the brick that pass stages
@@ -756,7 +752,6 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
     // selection, brick-boundary states) -> selection -> WENO and the limiter's
     // exact sequence into rows -> fused reconstruction + Riemann + divergence +
     // RK update
-    check(launch_zero(counter_ + 2, sizeof(int), stream_), "clear row count");
     timed("linear", [&] {
       return launch_linear_surf(dim, nq, Uin, wi, thNew, props_, grid_, parW_, ppList_, counter_ + 1, SB_, sb_,
                                 stream_, lrn ? &la : nullptr);
@@ -987,8 +982,8 @@ int Solver::takeStep() {
   stateInCur_ = false;
   stagePos_ = 0;
   for (int nT = 0; nT < cfg_.rejectionLimit; nT++) {
-    check(launch_zero(vmax_, sizeof(unsigned long long), stream_), "clear vmax");
-    if (nT > 0) {
+    if (nT > 0) {  // the speeds of the re-primed stage count for the attempt
+      check(launch_zero(vmax_, sizeof(unsigned long long), stream_), "clear vmax");
       RKArgs a{};
       a.mode = RK_PRIME;
       a.K = K_;
@@ -997,7 +992,7 @@ int Solver::takeStep() {
     }
     timed("stage_pre", [&] {
       return launch_stage_pre(nv_, Uprev_, K_, U_[cur_], Uhat_, Utmp_, rk_.beta[0] * dt,
-                              rk_.bhat[0] * dt, int(ncell_), stream_);
+                              rk_.bhat[0] * dt, int(ncell_), nT > 0 ? nullptr : vmax_, stream_);
     });
     for (int s = 1; s < rk_.nStages; s++) {
       RKArgs a{};
@@ -1029,10 +1024,7 @@ int Solver::takeStep() {
       a.vmaxBits = vmax_;
       pipeline(U_[cur_], a);
     }
-    check(launch_finalize(errPart_, posPart_, nPart_, redOut_, stream_), "finalize");
-    check(hipMemcpyAsync(hostRed_, redOut_, 2 * sizeof(double), hipMemcpyDeviceToHost, stream_), "read err");
-    check(hipMemcpyAsync(&hostRed_[2], vmax_, sizeof(double), hipMemcpyDeviceToHost, stream_), "read vmax");
-    check(hipMemcpyAsync(&hostRed_[3], counter_, sizeof(int), hipMemcpyDeviceToHost, stream_), "read count");
+    check(launch_finalize(errPart_, posPart_, nPart_, vmax_, counter_, hostRed_, stream_), "finalize");
     check(hipStreamSynchronize(stream_), "sync");
     const double errSum = hostRed_[0], posFlag = hostRed_[1];
     double maxVel;
@@ -1151,8 +1143,7 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
     check(hipStreamSynchronize(stream_), "sync");
     return;
   }
-  check(launch_zero(counter_, 2 * sizeof(int), stream_), "clear counters");
-  check(launch_cell_props(dim, Uin, props_, grid_, stream_), "cell_props");
+  check(launch_cell_props(dim, Uin, props_, grid_, counter_, stream_), "cell_props");
   check(launch_linear(dim, nq, nv_, Uin, FS_, WI_, thScratch, props_, grid_, faceW_, faceWT_, ppList_, counter_ + 1,
                       stream_, nullptr, sym_ ? parW_ : nullptr),
         "linear");
@@ -1172,10 +1163,9 @@ void Solver::advanceStages(int64_t n, double dtFixed) {
   stateInCur_ = false;
   for (int64_t it = 0; it < n; it++) {
     if (stagePos_ == 0) {
-      check(launch_zero(vmax_, sizeof(unsigned long long), stream_), "clear vmax");
       timed("stage_pre", [&] {
         return launch_stage_pre(nv_, Uprev_, K_, U_[cur_], Uhat_, Utmp_, rk_.beta[0] * dtFixed,
-                                rk_.bhat[0] * dtFixed, int(ncell_), stream_);
+                                rk_.bhat[0] * dtFixed, int(ncell_), vmax_, stream_);
       });
       stagePos_ = 1;
     }
@@ -1207,7 +1197,7 @@ void Solver::advanceStages(int64_t n, double dtFixed) {
       a.errPartial = errPart_;
       a.posPartial = posPart_;
       pipeline(U_[cur_], a);
-      check(launch_finalize(errPart_, posPart_, nPart_, redOut_, stream_), "finalize");
+      check(launch_finalize(errPart_, posPart_, nPart_, vmax_, counter_, hostRed_, stream_), "finalize");
       std::swap(Uprev_, U_[cur_]);
       time += dtFixed;
       nTS++;
@@ -1345,7 +1335,7 @@ void Solver::uploadWeights() {
                          nCell ? wts_.cell.data() : nullptr);
     check(hipMemcpy(faceWC_, wc.data(), wc.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
   }
-  if (parW_) {  // parity coefficients of the full-stencil face weights, [type][C]
+  if (parW_) {  // parity coefficients of the full-stencil face (and interior) weights, [type][C]
     std::vector<double> pw;
     sym_ = wts_.dim == 3 ? parity_face_list<3>(wts_.nq, wts_.face.data(), pw)
                          : parity_face_list<2>(wts_.nq, wts_.face.data(), pw);

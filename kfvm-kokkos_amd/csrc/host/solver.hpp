@@ -182,9 +182,9 @@ class Solver {
   void evalFlowStats();
   double *faceW_ = nullptr, *derivW_ = nullptr, *faceWT_ = nullptr, *faceWS_ = nullptr, *derivWS_ = nullptr;
   double *faceWC_ = nullptr;  // Euler WENO: compact face + derivative weights (compact_weno_weights)
-  double *errPart_ = nullptr, *posPart_ = nullptr, *redOut_ = nullptr;
+  double *errPart_ = nullptr, *posPart_ = nullptr;
   unsigned long long *vmax_ = nullptr;
-  double *hostRed_ = nullptr;  // pinned: [err, pos, vmax bits, counter]
+  double *hostRed_ = nullptr;  // pinned: [err, pos, vmax bits, counter], written by k_finalize
   int nPart_ = 0;
   bool lastRhsFull_ = false;  // the last RHS evaluation ran WENO on every cell
   bool stateInCur_ = false;  // last step was not accepted: the solution is in U_[cur_]
