@@ -34,7 +34,8 @@ CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall"]
 
 HOST_CXX = ["common.cpp", "weights.cpp", "problems.cpp", "writer.cpp"]
 HOST_HIP = ["solver.cpp", "indicator.cpp", "capi.cpp"]
-DEVICE = ["inst_mhd_d3q3.hip", "inst_mhd_d3q2.hip", "inst_d3q3.hip", "inst_d3q2.hip", "inst_mhd_d2q3.hip",
+DEVICE = ["inst_mhd_dense_d3q3.hip", "inst_mhd_dense_d3q2.hip", "inst_mhd_dense_d2q3.hip", "inst_mhd_dense_d2q2.hip",
+          "inst_mhd_d3q3.hip", "inst_mhd_d3q2.hip", "inst_d3q3.hip", "inst_d3q2.hip", "inst_mhd_d2q3.hip",
           "inst_mhd_d2q2.hip", "inst_d2q3.hip", "inst_d2q2.hip", "dispatch.hip", "noalloc.hip"]
 
 

@@ -219,9 +219,13 @@ hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid 
 // (PI = mhd_interior_pass_points).  Cells whose states violate a limiter
 // bound are appended to ppList (count in *ppCount, zeroed by the caller) for
 // launch_mhd_pp; the others get theta = 1.  WI may be null (learned selection).
+// PW (may be null): the parity coefficients of mirror-symmetric weights, face
+// points [type][C] then interior points [type][C]; used for the shapes of
+// mhd_parity (a thread would keep 18 points of six sums with the 3D 3x3 rule).
+constexpr bool mhd_parity(int dim, int nq) { return dim == 2 || nq == 2; }
 hipError_t launch_mhd_linear(int dim, int nq, const double *U, double *FS, double *SRC, double *WI,
                              double *thetaNew, double *spd, const double *props, const Grid &g, const double *WT,
-                             int *ppList, int *ppCount, hipStream_t s);
+                             const double *PW, int *ppList, int *ppCount, hipStream_t s);
 hipError_t launch_mhd_select(int dim, int nq, const double *U, const double *WI, const double *theta,
                              double *wflag, int *list, int *counter, double wThresh, const Grid &g,
                              hipStream_t s);

@@ -101,8 +101,8 @@ hipError_t launch_mhd_props(int dim, const double *U, double *props, const Grid 
 }
 hipError_t launch_mhd_linear(int dim, int nq, const double *U, double *FS, double *SRC, double *WI,
                              double *thetaNew, double *spd, const double *props, const Grid &g, const double *WT,
-                             int *ppList, int *ppCount, hipStream_t s) {
-  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::linear(U, FS, SRC, WI, thetaNew, spd, props, g, WT, ppList, ppCount, s));
+                             const double *PW, int *ppList, int *ppCount, hipStream_t s) {
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::linear(U, FS, SRC, WI, thetaNew, spd, props, g, WT, PW, ppList, ppCount, s));
 }
 hipError_t launch_mhd_select(int dim, int nq, const double *U, const double *WI, const double *theta,
                              double *wflag, int *list, int *counter, double wThresh, const Grid &g,

@@ -63,6 +63,14 @@ struct Launch {
                             hipStream_t s, int shape);
 };
 
+// The dense GLM-MHD linear pass, in units of its own (inst_mhd_dense_*.hip).
+template <int D, int NQ>
+struct LaunchMhdDense {
+  static hipError_t linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew, double *spd,
+                               const double *props, const Grid &g, const double *WT, int *ppList, int *ppCount,
+                               hipStream_t s);
+};
+
 // The GLM-MHD kernels, in translation units of their own (inst_mhd_*.hip).
 template <int D, int NQ>
 struct LaunchMhd {
@@ -70,7 +78,7 @@ struct LaunchMhd {
   static hipError_t props(const double *U, double *props, const Grid &g, int *counter, unsigned long long *chBits,
                           hipStream_t s);
   static hipError_t linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew, double *spd,
-                               const double *props, const Grid &g, const double *WT, int *ppList, int *ppCount,
+                               const double *props, const Grid &g, const double *WT, const double *PW, int *ppList, int *ppCount,
                                hipStream_t s);
   static hipError_t select(const double *U, const double *WI, const double *theta, double *wflag,
                                int *list, int *counter, double wThresh, const Grid &g, hipStream_t s);
@@ -88,6 +96,10 @@ extern template struct Launch<2, 2>;
 extern template struct Launch<2, 3>;
 extern template struct Launch<3, 2>;
 extern template struct Launch<3, 3>;
+extern template struct LaunchMhdDense<2, 2>;
+extern template struct LaunchMhdDense<2, 3>;
+extern template struct LaunchMhdDense<3, 2>;
+extern template struct LaunchMhdDense<3, 3>;
 extern template struct LaunchMhd<2, 2>;
 extern template struct LaunchMhd<2, 3>;
 extern template struct LaunchMhd<3, 2>;

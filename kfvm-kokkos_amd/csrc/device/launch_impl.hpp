@@ -174,12 +174,22 @@ hipError_t LaunchMhd<D, NQ>::props(const double *U, double *props, const Grid &g
 
 template <int D, int NQ>
 hipError_t LaunchMhd<D, NQ>::linear(const double *U, double *FS, double *SRC, double *WI, double *thetaNew,
-                                     double *spd, const double *props, const Grid &g, const double *WT,
-                                     int *ppList, int *ppCount, hipStream_t s) {
+                                    double *spd, const double *props, const Grid &g, const double *WT,
+                                    const double *PW, int *ppList, int *ppCount, hipStream_t s) {
   // WI null: the learned selection does not read the KXRCF indicator
-  hipLaunchKernelGGL((dev::k_mhd_linear<D, NQ>), dim3(bricks(g)), dim3(dev::MBox<D>::NT), 0, s, U, FS, SRC,
-                     WI, thetaNew, spd, props, g, WT, ppList, ppCount);
-  return hipGetLastError();
+  if constexpr (mhd_parity(D, NQ)) {
+    if (PW) {
+      const dim3 nb(bricks(g)), nt(dev::MBox<D>::NT);
+      if (WI)
+        hipLaunchKernelGGL((dev::k_mhd_linear_par<D, NQ, true>), nb, nt, 0, s, U, FS, SRC, WI, thetaNew, spd, props, g,
+                           PW, ppList, ppCount);
+      else
+        hipLaunchKernelGGL((dev::k_mhd_linear_par<D, NQ, false>), nb, nt, 0, s, U, FS, SRC, WI, thetaNew, spd, props,
+                           g, PW, ppList, ppCount);
+      return hipGetLastError();
+    }
+  }
+  return LaunchMhdDense<D, NQ>::linear(U, FS, SRC, WI, thetaNew, spd, props, g, WT, ppList, ppCount, s);
 }
 
 template <int D, int NQ>

@@ -48,6 +48,12 @@ __device__ __forceinline__ void static_for(F &&f) {
 }
 #define KFVM_INLINE __attribute__((always_inline))
 
+// The value is formed here: the compiler would otherwise sink a sum, a test or a
+// maximum to its last use and keep all its terms in registers until then (724 B
+// of scratch a thread instead of none in 3D).
+__device__ __forceinline__ void keep_here(double &x) { asm volatile("" : "+v"(x)); }
+__device__ __forceinline__ void keep_here(int &x) { asm volatile("" : "+v"(x)); }
+
 // The butterflies over the stencil values of one variable, in place.
 template <int D>
 __device__ __forceinline__ void parity_transform(double (&t)[SInfo<D>::C]) {

@@ -1010,6 +1010,7 @@ __global__ __launch_bounds__(BLK, NV == 9 ? (D == 3 && NQ == 3 ? 1 : 2) : 3) voi
 #include "parity5.hpp"
 #include "points5.hpp"
 #include "mhd.hpp"
+#include "parity9.hpp"
 #include "indicator.hpp"
 
 namespace kfvm {

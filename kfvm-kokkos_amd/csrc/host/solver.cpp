@@ -150,7 +150,10 @@ void Solver::setup() {
     const char *ev = std::getenv("KFVM_FUSED");
     fusedWanted_ = fused_flux(cfg_.dim, cfg_.nQuad) && !(ev && std::string(ev) == "0");
     pos_ = dalloc<int>(nc, "row of each cell");
-    parW_ = dalloc<double>(size_t(parity_face_types(cfg_.dim, cfg_.nQuad)) * wts_.C, "parity weights");
+  }
+  if (nv_ != 1) {
+    const int types = parity_face_types(cfg_.dim, cfg_.nQuad) + (nv_ == 9 ? parity_cell_types(cfg_.dim, cfg_.nQuad) : 0);
+    parW_ = dalloc<double>(size_t(types) * wts_.C, "parity weights");
   }
   WI_ = dalloc<double>(fs_elems(nc, int(FQ)), "indicator");
   props_ = dalloc<double>(nc * 2, "cell properties");
@@ -674,7 +677,7 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
     const bool lrn = learned_ && !forcePlain_;
     timed("linear", [&] {
       return launch_mhd_linear(dim, nq, Uin, FS_, SRC_, lrn ? nullptr : WI_, thNew, spd_, props_, grid_, mhdWT_,
-                               ppList_, counter_ + 1, stream_);
+                               sym_ ? parW_ : nullptr, ppList_, counter_ + 1, stream_);
     });
     if (lrn) {
       timed("select", [&] {
@@ -1129,9 +1132,8 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
   if (!FSlin_) FSlin_ = dalloc<double>(fsBytes / sizeof(double), "linear face states");
   if (nv_ == 9) {
     // labels compare the linear face states with the limited WENO ones
-    check(launch_zero(counter_, 2 * sizeof(int), stream_), "clear counters");
-    check(launch_mhd_props(dim, Uin, props_, grid_, stream_), "mhd_props");
-    check(launch_mhd_linear(dim, nq, Uin, FS_, SRC_, nullptr, thScratch, spd_, props_, grid_, mhdWT_, ppList_,
+    check(launch_mhd_props(dim, Uin, props_, grid_, counter_, chBits_, stream_), "mhd_props");
+    check(launch_mhd_linear(dim, nq, Uin, FS_, SRC_, nullptr, thScratch, spd_, props_, grid_, mhdWT_, sym_ ? parW_ : nullptr, ppList_,
                             counter_ + 1, stream_),
           "mhd_linear");
     check(hipMemcpyAsync(FSlin_, FS_, fsBytes, hipMemcpyDeviceToDevice, stream_), "copy linear states");
@@ -1339,6 +1341,12 @@ void Solver::uploadWeights() {
     std::vector<double> pw;
     sym_ = wts_.dim == 3 ? parity_face_list<3>(wts_.nq, wts_.face.data(), pw)
                          : parity_face_list<2>(wts_.nq, wts_.face.data(), pw);
+    if (nv_ == 9 && sym_) {
+      const size_t nf = pw.size();
+      pw.resize(nf + size_t(parity_cell_types(wts_.dim, wts_.nq)) * C);
+      sym_ = wts_.dim == 3 ? parity_coefficients<3>(wts_.nq, -1, wts_.cell.data(), pw.data() + nf)
+                           : parity_coefficients<2>(wts_.nq, -1, wts_.cell.data(), pw.data() + nf);
+    }
     if (sym_) check(hipMemcpy(parW_, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
     fused_ = fusedWanted_ && sym_;
     pathBuffers();

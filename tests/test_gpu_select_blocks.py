@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dim,nq,n", [
     (2, 2, (31, 33, 1)), (2, 2, (32, 32, 1)), (2, 2, (41, 25, 1)), (2, 3, (41, 50, 1)),
-    (3, 2, (11, 13, 7)), (3, 3, (7, 73, 1)), (3, 3, (8, 8, 8)), (3, 3, (27, 19, 1)),
+    (3, 2, (11, 13, 7)), (3, 3, (7, 37, 2)), (3, 3, (8, 8, 8)), (3, 3, (9, 19, 3)),
 ])
 def test_selected_cells_and_rhs(dim, nq, n):
     import kfvm_amd
