@@ -16,6 +16,7 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <thread>
 
 #include <rocprofiler-sdk-roctx/roctx.h>
 
@@ -604,6 +605,7 @@ void Solver::release() noexcept {
   for (void *p : bufs)
     if (p) (void)hipFree(p);
   if (hostRed_) (void)hipHostFree(hostRed_);
+  if (pin_) (void)hipHostFree(pin_);
   if (sHost_) (void)hipHostFree(sHost_);
   if (sMaskHost_) (void)hipHostFree(sMaskHost_);
   if (stream_) (void)hipStreamDestroy(stream_);
@@ -1271,26 +1273,73 @@ int64_t Solver::solve() {
   return n;
 }
 
-void Solver::getState(double *host) const {
-  const double *src = stateInCur_ ? U_[cur_] : Uprev_;
+// A large device array into pageable host memory: worker threads each take
+// every n-th chunk through a pinned buffer of their own, so that the DMA runs
+// at the link's rate while the host copies, and the first touch of fresh pages
+// (most of the time of one hipMemcpy: 64 ms for a 256^3 Euler state), are spread
+// over the threads.  The pinned buffers are the solver's, made by its first
+// large copy.
+void Solver::copyToHost(void *dst, const void *src, size_t bytes) const {
   check(hipStreamSynchronize(stream_), "sync");
-  check(hipMemcpy(host, src, size_t(ncell_) * nv_ * sizeof(double), hipMemcpyDeviceToHost), "get state");
+  constexpr size_t kChunk = size_t(2) << 20;
+  const size_t chunks = (bytes + kChunk - 1) / kChunk;
+  const unsigned nt = unsigned(std::min<size_t>({size_t(8), chunks / 4, size_t(std::thread::hardware_concurrency())}));
+  if (nt < 2) {
+    check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "copy to host");
+    return;
+  }
+  int dev = 0;
+  check(hipGetDevice(&dev), "hipGetDevice");
+  std::lock_guard<std::mutex> lock(pinMutex_);  // one copy at a time uses the buffers
+  if (!pin_ && hipHostMalloc((void **)&pin_, 8 * kChunk, hipHostMallocDefault) != hipSuccess) {
+    pin_ = nullptr;
+    (void)hipGetLastError();
+    check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "copy to host");
+    return;
+  }
+  std::vector<hipError_t> err(nt, hipSuccess);
+  std::vector<std::thread> th;
+  auto work = [&](unsigned t) {
+    hipError_t e = hipSetDevice(dev);
+    hipEvent_t ev = nullptr;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    char *const buf = pin_ + t * kChunk;
+    for (size_t c = t; c < chunks && e == hipSuccess; c += nt) {
+      const size_t off = c * kChunk, n = std::min(kChunk, bytes - off);
+      e = hipMemcpyAsync(buf, static_cast<const char *>(src) + off, n, hipMemcpyDeviceToHost, stream_);
+      if (e == hipSuccess) e = hipEventRecord(ev, stream_);
+      if (e == hipSuccess) e = hipEventSynchronize(ev);
+      if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + off, buf, n);
+    }
+    if (ev) (void)hipEventDestroy(ev);
+    err[t] = e;
+  };
+  unsigned started = 0;
+  try {
+    for (; started < nt; started++) th.emplace_back(work, started);
+  } catch (...) {  // no more threads: their chunks are copied here
+  }
+  for (auto &t : th) t.join();
+  for (unsigned t = started; t < nt; t++) work(t);
+  (void)hipStreamSynchronize(stream_);  // no copy into the buffers is in flight, whatever failed
+  for (hipError_t e : err) check(e, "copy to host");
+}
+
+void Solver::getState(double *host) const {
+  copyToHost(host, stateInCur_ ? U_[cur_] : Uprev_, size_t(ncell_) * nv_ * sizeof(double));
 }
 void Solver::setState(const double *host) {
   const size_t bytes = size_t(ncell_) * nv_ * sizeof(double);
   check(hipStreamSynchronize(stream_), "sync");
   check(hipMemcpy(Uprev_, host, bytes, hipMemcpyHostToDevice), "set state");
-  check(hipMemcpy(U_[cur_], host, bytes, hipMemcpyHostToDevice), "set state");
+  check(hipMemcpyAsync(U_[cur_], Uprev_, bytes, hipMemcpyDeviceToDevice, stream_), "set state");
+  check(hipStreamSynchronize(stream_), "set state");  // callers may read it from a stream of their own
   stateInCur_ = false;
 }
-void Solver::getRHS(double *host) const {
-  check(hipStreamSynchronize(stream_), "sync");
-  check(hipMemcpy(host, K_, size_t(ncell_) * nv_ * sizeof(double), hipMemcpyDeviceToHost), "get rhs");
-}
+void Solver::getRHS(double *host) const { copyToHost(host, K_, size_t(ncell_) * nv_ * sizeof(double)); }
 void Solver::getFlags(double *host) const {
-  check(hipStreamSynchronize(stream_), "sync");
-  check(hipMemcpy(host, wflag_, size_t(ncell_) * sizeof(double), hipMemcpyDeviceToHost), "get flags");
-  check(hipMemcpy(host + ncell_, theta_[th_], size_t(ncell_) * sizeof(double), hipMemcpyDeviceToHost), "get flags");
+  copyToHost(host, wflag_, size_t(ncell_) * sizeof(double));
+  copyToHost(host + ncell_, theta_[th_], size_t(ncell_) * sizeof(double));
 }
 void Solver::setFlags(const double *host) {
   check(hipStreamSynchronize(stream_), "sync");

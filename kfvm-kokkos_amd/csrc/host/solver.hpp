@@ -5,6 +5,7 @@
 //   Solver::TakeStep src/Solver.cpp:188-343    Solver::evalRHS  src/Solver.cpp:410-530
 #pragma once
 
+#include <mutex>
 #include <hip/hip_runtime.h>
 
 #include <map>
@@ -132,6 +133,7 @@ class Solver {
   void pipeline(const double *Uin, const RKArgs &a);
   void pipelineMhd(const double *Uin, const RKArgs &a);
   void uploadWeights();
+  void copyToHost(void *dst, const void *src, size_t bytes) const;
   void pathBuffers();
   // 3D Euler with the learned selection keeps one order of operations
   // (points5.hpp): its choice of cells reads the rounding of the state
@@ -185,6 +187,8 @@ class Solver {
   double *errPart_ = nullptr, *posPart_ = nullptr;
   unsigned long long *vmax_ = nullptr;
   double *hostRed_ = nullptr;  // pinned: [err, pos, vmax bits, counter], written by k_finalize
+  mutable char *pin_ = nullptr;  // pinned chunks of copyToHost
+  mutable std::mutex pinMutex_;
   int nPart_ = 0;
   bool lastRhsFull_ = false;  // the last RHS evaluation ran WENO on every cell
   bool stateInCur_ = false;  // last step was not accepted: the solution is in U_[cur_]
