@@ -190,6 +190,9 @@ hipError_t launch_select(int dim, int nq, const double *U, const double *WI, con
 // then [SUB][I] derivative weights (SUB = C + Cc + B*Cb, substencils back to
 // back; compact_weno_weights), DWS is not read.  WS (Euler, may be null): compact staging
 // [(F*Q*5)][cap] for the first cap listed cells, shared with launch_weno_post.
+// WP (may be null; also launch_mhd_weno's): the mirror-symmetric form of the
+// weights (host/parity_weno.hpp), which then takes the place of the dense
+// tables; the grid must have fewer than 2^29 cells (32-bit byte offsets).
 // Compact WENO weight table (see launch_weno) from the reference layouts
 // face [nSub][F*Q][C] and deriv [nSub][I][C]; out has SUB*(F*Q + I) doubles,
 // then, with nCell > 0 (GLM-MHD), SUB*nCell rows of the interior-point
@@ -199,7 +202,7 @@ void compact_weno_weights(int dim, int fq, int nI, const double *face, const dou
 hipError_t launch_weno(int dim, int nq, int nv, const double *U, double *FS, double *thetaNew,
                        const Grid &g, const double *FW, const double *DW, const double *FWS,
                        const double *DWS, const int *list, const int *counter, double *WS, int cap,
-                       hipStream_t s);
+                       const double *WP, hipStream_t s);
 // Euler: back to conserved variables and the positivity limiter on the
 // listed cells (in WS for the first cap of them, then copied to FS).
 hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double *thetaNew,
@@ -237,7 +240,7 @@ hipError_t launch_mhd_select(int dim, int nq, const double *U, const double *WI,
 hipError_t launch_mhd_weno(int dim, int nq, const double *U, double *FS, double *SRC, const Grid &g,
                            const double *FT, const double *DT, const double *CT, const int *list,
                            const int *counter, double *thetaNew, double *spd, const double *props,
-                           const double *WC, hipStream_t s);
+                           const double *WC, const double *WP, hipStream_t s);
 // The limiter's exact sequence on the listed cells whose WENO flag is 0.
 hipError_t launch_mhd_pp(int dim, int nq, const double *U, double *FS, double *SRC, double *thetaNew,
                          double *spd, const double *props, const double *wflag, const Grid &g, const int *list,

@@ -81,11 +81,11 @@ void compact_weno_weights(int dim, int fq, int nI, const double *face, const dou
 hipError_t launch_weno(int dim, int nq, int nv, const double *U, double *FS, double *thetaNew,
                        const Grid &g, const double *FW, const double *DW, const double *FWS,
                        const double *DWS, const int *list, const int *counter, double *WS, int cap,
-                       hipStream_t s) {
+                       const double *WP, hipStream_t s) {
   if (nv != 5 && nv != 1) return hipErrorInvalidValue;
   if (WS && cap < 0) return hipErrorInvalidValue;
   (void)DWS;
-  KFVM_SELECT(dim, nq, L::weno(nv, U, FS, thetaNew, g, FW, DW, list, counter, WS, cap, nv == 5 ? FWS : nullptr, s));
+  KFVM_SELECT(dim, nq, L::weno(nv, U, FS, thetaNew, g, FW, DW, list, counter, WS, cap, nv == 5 ? FWS : nullptr, WP, s));
 }
 
 hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double *thetaNew,
@@ -112,8 +112,8 @@ hipError_t launch_mhd_select(int dim, int nq, const double *U, const double *WI,
 hipError_t launch_mhd_weno(int dim, int nq, const double *U, double *FS, double *SRC, const Grid &g,
                            const double *FT, const double *DT, const double *CT, const int *list,
                            const int *counter, double *thetaNew, double *spd, const double *props,
-                           const double *WC, hipStream_t s) {
-  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::weno(U, FS, SRC, g, FT, DT, CT, list, counter, thetaNew, spd, props, WC, s));
+                           const double *WC, const double *WP, hipStream_t s) {
+  KFVM_SELECT_OF(LaunchMhd, dim, nq, L::weno(U, FS, SRC, g, FT, DT, CT, list, counter, thetaNew, spd, props, WC, WP, s));
 }
 hipError_t launch_mhd_pp(int dim, int nq, const double *U, double *FS, double *SRC, double *thetaNew,
                          double *spd, const double *props, const double *wflag, const Grid &g, const int *list,

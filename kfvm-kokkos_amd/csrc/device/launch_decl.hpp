@@ -25,7 +25,7 @@ struct Launch {
                            hipStream_t s);
   static hipError_t weno(int nv, const double *U, double *FS, double *thetaNew, const Grid &g,
                          const double *FW, const double *DW, const int *list, const int *counter,
-                         double *WS, int cap, const double *WC, hipStream_t s);
+                         double *WS, int cap, const double *WC, const double *WP, hipStream_t s);
   // ---- fused path (Euler, sparse WENO)
   static hipError_t linear_surf(const double *U, double *WI, double *thetaNew, const double *props,
                                 const Grid &g, const double *PW, int *ppList, int *ppCount, double *SB,
@@ -84,7 +84,8 @@ struct LaunchMhd {
                                int *list, int *counter, double wThresh, const Grid &g, hipStream_t s);
   static hipError_t weno(const double *U, double *FS, double *SRC, const Grid &g, const double *FT,
                              const double *DT, const double *CT, const int *list, const int *counter,
-                             double *thetaNew, double *spd, const double *props, const double *WC, hipStream_t s);
+                             double *thetaNew, double *spd, const double *props, const double *WC, const double *WP,
+                             hipStream_t s);
   static hipError_t pp(const double *U, double *FS, double *SRC, double *thetaNew, double *spd,
                            const double *props, const double *wflag, const Grid &g, const int *list,
                            const int *count, hipStream_t s);

@@ -11,6 +11,10 @@
 
 namespace kfvm {
 
+// Workgroups of k_weno_par: the list's length is not known here, so the grid is
+// bounded by what fills the chip several times over and strides.
+inline unsigned weno_par_blocks(const Grid &g) { return std::min<unsigned>((unsigned(g.ncell) + 63) / 64, 2048u); }
+
 template <int D, int NQ>
 unsigned Launch<D, NQ>::bricks(const Grid &g) {
   using Bx = dev::RBox<D>;
@@ -61,15 +65,22 @@ hipError_t Launch<D, NQ>::select(const double *U, const double *WI, const double
 template <int D, int NQ>
 hipError_t Launch<D, NQ>::weno(int nv, const double *U, double *FS, double *thetaNew, const Grid &g,
                                const double *FW, const double *DW, const int *list, const int *counter,
-                               double *WS, int cap, const double *WC, hipStream_t s) {
+                               double *WS, int cap, const double *WC, const double *WP, hipStream_t s) {
   if (nv == 5) {
+    // KFVM_WENO_SCALAR=1 (read at every launch) runs the scalar kernel
+    // instead: the others are compared with it in the tests
+    const char *ev = std::getenv("KFVM_WENO_SCALAR");
+    const bool scalar = ev && ev[0] == '1';
+    if (WP && !scalar) {
+      using K = dev::WenoPar<D, NQ, 5>;
+      hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 5>), dim3(weno_par_blocks(g)), dim3(K::NT), 0, s, U, FS, nullptr, g,
+                         WP, list, counter, WS, WS ? cap : 0);
+      return hipGetLastError();
+    }
     // persistent: every workgroup stages the weights once, then strides over the list
     if (!WC) return hipErrorInvalidValue;
     if constexpr (dev::WenoMfma<D, NQ>::USE) {
-      // KFVM_WENO_SCALAR=1 (read at every launch) runs the scalar kernel
-      // instead: the two are compared in the tests
-      const char *ev = std::getenv("KFVM_WENO_SCALAR");
-      if (!(ev && ev[0] == '1')) {
+      if (!scalar) {
         constexpr int cellsPerBlock = 16 * dev::WenoMfma<D, NQ>::WPB;
         const unsigned nb = std::min<unsigned>(unsigned((g.ncell + cellsPerBlock - 1) / cellsPerBlock), 2048u);
         hipLaunchKernelGGL((dev::k_wenorec5_mfma<D, NQ>), dim3(nb), dim3(dev::BLK), 0, s, U, FS, g, WC, list,
@@ -205,13 +216,17 @@ template <int D, int NQ>
 hipError_t LaunchMhd<D, NQ>::weno(const double *U, double *FS, double *SRC, const Grid &g, const double *FT,
                                    const double *DT, const double *CT, const int *list, const int *counter,
                                    double *thetaNew, double *spd, const double *props, const double *WC,
-                                   hipStream_t s) {
+                                   const double *WP, hipStream_t s) {
   // weights in LDS: persistent (every workgroup stages the table once, then strides over the list)
   constexpr bool lds = dev::MWenoLds<D, NQ>::USE;
   if (lds && !WC) return hipErrorInvalidValue;
   const unsigned nb = std::min<unsigned>(unsigned((g.ncell + dev::MCPB - 1) / dev::MCPB), lds ? 2048u : 1u << 16);
-  hipLaunchKernelGGL((dev::k_mhd_wenorec<D, NQ>), dim3(nb), dim3(dev::BLK), 0, s, U, FS, SRC, g, FT, DT, CT,
-                     list, counter, WC);
+  if (WP)
+    hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 9>), dim3(weno_par_blocks(g)), dim3(dev::WenoPar<D, NQ, 9>::NT), 0, s,
+                       U, FS, SRC, g, WP, list, counter, nullptr, 0);
+  else
+    hipLaunchKernelGGL((dev::k_mhd_wenorec<D, NQ>), dim3(nb), dim3(dev::BLK), 0, s, U, FS, SRC, g, FT, DT, CT,
+                       list, counter, WC);
   const unsigned np = std::min<unsigned>(stage_blocks(g.ncell), 1u << 16);
   if (list)
     hipLaunchKernelGGL((dev::k_mhd_weno_post<D, NQ>), dim3(np), dim3(dev::BLK), 0, s, U, FS, SRC, g, list,

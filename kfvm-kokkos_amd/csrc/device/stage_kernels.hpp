@@ -33,6 +33,7 @@
 #include <utility>
 
 #include "../host/parity.hpp"
+#include "../host/parity_weno.hpp"
 #include "../host/stencil_geom.hpp"
 #include "device_api.hpp"
 #include "physics.hpp"
@@ -1011,6 +1012,7 @@ __global__ __launch_bounds__(BLK, NV == 9 ? (D == 3 && NQ == 3 ? 1 : 2) : 3) voi
 #include "points5.hpp"
 #include "mhd.hpp"
 #include "parity9.hpp"
+#include "weno_par.hpp"
 #include "indicator.hpp"
 
 namespace kfvm {

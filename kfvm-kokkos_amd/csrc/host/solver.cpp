@@ -22,6 +22,7 @@
 
 #include "problems.hpp"
 #include "parity.hpp"
+#include "parity_weno.hpp"
 #include "stencil_geom.hpp"
 
 namespace kfvm {
@@ -155,6 +156,10 @@ void Solver::setup() {
   if (nv_ != 1) {
     const int types = parity_face_types(cfg_.dim, cfg_.nQuad) + (nv_ == 9 ? parity_cell_types(cfg_.dim, cfg_.nQuad) : 0);
     parW_ = dalloc<double>(size_t(types) * wts_.C, "parity weights");
+    const bool cells = nv_ == 9;
+    const int nw = cfg_.dim == 3 ? (cfg_.nQuad == 2 ? weno_parity_size<3, 2>(cells) : weno_parity_size<3, 3>(cells))
+                                 : (cfg_.nQuad == 2 ? weno_parity_size<2, 2>(cells) : weno_parity_size<2, 3>(cells));
+    wenoP_ = dalloc<double>(size_t(nw), "WENO parity weights");
   }
   WI_ = dalloc<double>(fs_elems(nc, int(FQ)), "indicator");
   props_ = dalloc<double>(nc * 2, "cell properties");
@@ -597,7 +602,7 @@ void Solver::release() noexcept {
   } catch (...) {
   }
   void *bufs[] = {SRC_, cellW_, cellWS_, diffM_, chBits_, U_[0], U_[1], Uprev_, Uhat_, K_, Utmp_, FS_, WI_, props_, theta_[0], theta_[1], wflag_, list_, counter_, ppList_,
-                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
+                  faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, wenoP_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
   if (stream_) (void)hipStreamSynchronize(stream_);
   for (auto &kv : graphs_)
     if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
@@ -694,7 +699,7 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
     }
     timed("weno", [&] {
       return launch_mhd_weno(dim, nq, Uin, FS_, SRC_, grid_, faceWS_, derivWS_, cellWS_, list_, counter_, thNew,
-                             spd_, props_, faceWC_, stream_);
+                             spd_, props_, faceWC_, wenoWeights(true), stream_);
     });
     timed("pp", [&] {
       return launch_mhd_pp(dim, nq, Uin, FS_, SRC_, thNew, spd_, props_, wflag_, grid_, ppList_, counter_ + 1,
@@ -703,7 +708,7 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
   } else {
     timed("weno", [&] {
       return launch_mhd_weno(dim, nq, Uin, FS_, SRC_, grid_, faceWS_, derivWS_, cellWS_, nullptr, nullptr, thNew,
-                             spd_, props_, faceWC_, stream_);
+                             spd_, props_, faceWC_, wenoWeights(false), stream_);
     });
     useSparseWeno = cfg_.wenoThresh > 0.0;
   }
@@ -768,7 +773,7 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
       });
     timed("weno", [&] {
       return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_, counter_,
-                         FS_, cap, stream_);
+                         FS_, cap, wenoWeights(true), stream_);
     });
     timed("weno_post", [&] {
       return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, FS_, cap, stream_);
@@ -798,7 +803,7 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
         });
       timed("weno", [&] {
         return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_,
-                           counter_, WS_, cap, stream_);
+                           counter_, WS_, cap, wenoWeights(true), stream_);
       });
       timed("weno_post", [&] {
         return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, WS_, cap, stream_);
@@ -810,7 +815,7 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   } else {
     timed("weno", [&] {
       return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, nullptr,
-                         nullptr, nullptr, 0, stream_);
+                         nullptr, nullptr, 0, wenoWeights(false), stream_);
     });
     if (hydro)
       timed("weno_post", [&] {
@@ -1140,7 +1145,7 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
           "mhd_linear");
     check(hipMemcpyAsync(FSlin_, FS_, fsBytes, hipMemcpyDeviceToDevice, stream_), "copy linear states");
     check(launch_mhd_weno(dim, nq, Uin, FS_, SRC_, grid_, faceWS_, derivWS_, cellWS_, nullptr, nullptr, thScratch,
-                          spd_, props_, faceWC_, stream_),
+                          spd_, props_, faceWC_, wenoWeights(false), stream_),
           "mhd_weno");
     check(launch_labels(dim, nq, 9, Uin, FSlin_, FS_, float(tau), Y, grid_, stream_), "labels");
     check(launch_features(dim, 9, Uin, nullptr, X, grid_, stream_), "features");
@@ -1153,7 +1158,7 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
         "linear");
   check(hipMemcpyAsync(FSlin_, FS_, fsBytes, hipMemcpyDeviceToDevice, stream_), "copy linear states");
   check(launch_weno(dim, nq, nv_, Uin, FS_, thScratch, grid_, faceW_, derivW_, faceWC_, derivWS_, nullptr, nullptr,
-                    nullptr, 0, stream_),
+                    nullptr, 0, wenoWeights(false), stream_),
         "weno");
   check(launch_weno_post(dim, nq, Uin, FS_, thScratch, props_, grid_, nullptr, nullptr, nullptr, 0, stream_),
         "weno_post");
@@ -1398,6 +1403,15 @@ void Solver::uploadWeights() {
     }
     if (sym_) check(hipMemcpy(parW_, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
     fused_ = fusedWanted_ && sym_;
+    const double *cell = nv_ == 9 ? wts_.cell.data() : nullptr;
+    const double *face = wts_.face.data(), *der = wts_.deriv.data();
+    wenoSym_ = wts_.dim == 3 ? (wts_.nq == 2 ? weno_parity_list<3, 2>(face, der, cell, pw)
+                                             : weno_parity_list<3, 3>(face, der, cell, pw))
+                             : (wts_.nq == 2 ? weno_parity_list<2, 2>(face, der, cell, pw)
+                                             : weno_parity_list<2, 3>(face, der, cell, pw));
+    wenoSym_ = wenoSym_ && ncell_ < (int64_t(1) << 29);  // the kernel's byte offsets have 32 bits
+    if (wenoSym_)
+      check(hipMemcpy(wenoP_, pw.data(), pw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
     pathBuffers();
   }
   if (cellW_) {

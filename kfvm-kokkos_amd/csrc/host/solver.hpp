@@ -139,6 +139,13 @@ class Solver {
   // (points5.hpp): its choice of cells reads the rounding of the state
   bool pointOrder() const { return learned_ && nv_ == 5 && cfg_.dim == 3; }
   bool fusedNow() const { return fused_ && !noFuse_ && !pointOrder(); }
+  // Weights of k_weno_par, for a list or for every cell.  3D Euler with the
+  // learned selection, and with WENO on every cell, which a learned run that
+  // picks every cell equals, keep the kernel their order of sums comes from.
+  const double *wenoWeights(bool list) const {
+    const bool dense = nv_ == 5 && cfg_.dim == 3 && (!list || learned_);
+    return wenoSym_ && !dense ? wenoP_ : nullptr;
+  }
   bool noFuse_ = false;  // this evaluation's scratch only fits the unfused path
   double readSpeed();
   bool nadFails();
@@ -164,7 +171,7 @@ class Solver {
   // pass (surface planes); listed cells keep their states in rows of FS_.
   // sym_: the full-stencil weights are mirror-symmetric, parW_ their parity
   // coefficients [type][C]
-  bool fused_ = false, fusedWanted_ = false, sym_ = false;
+  bool fused_ = false, fusedWanted_ = false, sym_ = false, wenoSym_ = false;
   double *SB_ = nullptr, *parW_ = nullptr;
   Surf sb_{};
   double *props_ = nullptr;  // per-cell internal energy and sound speed [2][ncell]
@@ -183,6 +190,7 @@ class Solver {
   int statsRow_ = 0;             // next row of <basename>_stats.h5
   void evalFlowStats();
   double *faceW_ = nullptr, *derivW_ = nullptr, *faceWT_ = nullptr, *faceWS_ = nullptr, *derivWS_ = nullptr;
+  double *wenoP_ = nullptr;   // WENO weights in mirror-symmetric form (weno_parity_list)
   double *faceWC_ = nullptr;  // Euler WENO: compact face + derivative weights (compact_weno_weights)
   double *errPart_ = nullptr, *posPart_ = nullptr;
   unsigned long long *vmax_ = nullptr;
