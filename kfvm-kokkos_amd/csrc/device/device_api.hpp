@@ -301,10 +301,13 @@ hipError_t launch_logits(int dim, const float *X, const float *P, float *Z, int 
 hipError_t launch_train_grad(int dim, const float *X, const float *Y, const int *idx, int n, int nb,
                              uint64_t seed, const float *P, float posW, float *part, float *lossPart,
                              hipStream_t s);
+// The batch's gradient and loss; with ad.M also the Adam step.
+struct AdamArgs {
+  float *M, *Pbf, *m1, *m2;
+  float lr, b1, b2, eps, c1, c2;
+};
 hipError_t launch_train_reduce(const float *part, const float *lossPart, int nblk, int np, int nb, float *grad,
-                               float *loss, hipStream_t s);
-hipError_t launch_adam(float *M, float *Pbf, const float *grad, float *m1, float *m2, int np, float lr,
-                       float b1, float b2, float eps, float c1, float c2, hipStream_t s);
+                               float *loss, const AdamArgs &ad, hipStream_t s);
 hipError_t launch_nad(int dim, int nv, const double *Uold, const double *Unew, double fr, double fv,
                       double *nadFlag, int *count, const Grid &g, hipStream_t s);
 

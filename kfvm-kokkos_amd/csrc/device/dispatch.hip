@@ -230,15 +230,9 @@ hipError_t launch_train_grad(int dim, const float *X, const float *Y, const int 
   KFVM_SELECT(dim, 2, L::train_grad(X, Y, idx, n, nb, seed, P, posW, part, lossPart, s));
 }
 hipError_t launch_train_reduce(const float *part, const float *lossPart, int nblk, int np, int nb, float *grad,
-                               float *loss, hipStream_t s) {
-  hipLaunchKernelGGL(dev::k_train_reduce, dim3(stage_blocks(np)), dim3(dev::BLK), 0, s, part, lossPart, nblk, np,
-                     nb, grad, loss);
-  return hipGetLastError();
-}
-hipError_t launch_adam(float *M, float *Pbf, const float *grad, float *m1, float *m2, int np, float lr,
-                       float b1, float b2, float eps, float c1, float c2, hipStream_t s) {
-  hipLaunchKernelGGL(dev::k_adam, dim3(stage_blocks(np)), dim3(dev::BLK), 0, s, M, Pbf, grad, m1, m2, np, lr, b1,
-                     b2, eps, c1, c2);
+                               float *loss, const AdamArgs &ad, hipStream_t s) {
+  hipLaunchKernelGGL(dev::k_train_reduce, dim3(unsigned(np) / dev::TRB + 1), dim3(dev::TRB), 0, s, part, lossPart, nblk,
+                     np, nb, grad, loss, ad);
   return hipGetLastError();
 }
 hipError_t launch_nad(int dim, int nv, const double *Uold, const double *Unew, double fr, double fv,

@@ -600,7 +600,8 @@ __global__ __launch_bounds__(BLK) void k_labels(const double *__restrict__ U, co
 }
 
 // ------------------------------------------------------------------ training
-constexpr int TB = 64;  // samples per training block (one wave)
+constexpr int TB = 64;  // samples per training block (the lanes of a wave)
+constexpr int TW = 8;   // waves of a training block
 
 __device__ inline uint32_t mix32(uint64_t x) {
   x += 0x9E3779B97F4A7C15ull;
@@ -618,117 +619,119 @@ __device__ inline int batch_index(const int *__restrict__ idx, int b, int n, uin
 // Per-block partial gradient of the class-weighted logistic loss
 //   L_s = w_s * softplus(z_s (1 - 2 y_s)),  w_s = posW if y_s = 1 else 1,
 // over TB samples of a batch of nb: part[blk][NP] gradient sums, lossPart[blk].
+// A batch has only a few samples per CU, so what counts is the length of the
+// serial chain: the lanes are the samples, and the workgroup's TW waves split
+// the units of each layer, then the parameters.  Every sum keeps its order.
+// 8192 samples in 2D: 50 us with one wave per workgroup, 17 us with eight.
 template <int D>
-__global__ __launch_bounds__(TB) void k_train_grad(const float *__restrict__ X, const float *__restrict__ Y,
-                                                   const int *__restrict__ idx, int n, int nb,
-                                                   uint64_t seed, const float *__restrict__ P,
-                                                   float posW, float *__restrict__ part,
-                                                   float *__restrict__ lossPart) {
+__global__ __launch_bounds__(TB * TW) void k_train_grad(const float *__restrict__ X, const float *__restrict__ Y,
+                                                        const int *__restrict__ idx, int n, int nb,
+                                                        uint64_t seed, const float *__restrict__ P,
+                                                        float posW, float *__restrict__ part,
+                                                        float *__restrict__ lossPart) {
   using N = Net<D>;
+  constexpr int JW = N::H / TW;  // units of a wave
+  static_assert(N::H % TW == 0, "the waves split the units evenly");
   __shared__ float xs[TB][N::NIN + 1];
   __shared__ float h1s[TB][N::H + 1], h2s[TB][N::H + 1], d1s[TB][N::H + 1], d2s[TB][N::H + 1];
   __shared__ float dzs[TB], ls[TB];
-  const int t = threadIdx.x;
+  const int t = threadIdx.x % TB;
+  const int j0 = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / TB) * JW;
   const int b = blockIdx.x * TB + t;
   const bool live = b < nb;
   const int s = live ? batch_index(idx, b, n, seed) : 0;
   float x[N::NIN];
 #pragma unroll
-  for (int i = 0; i < N::NIN; i++) {
-    x[i] = live ? X[size_t(s) * N::NIN + i] : 0.0f;
-    xs[t][i] = x[i];
-  }
+  for (int i = 0; i < N::NIN; i++) x[i] = live ? X[size_t(s) * N::NIN + i] : 0.0f;
   const float y = live ? Y[s] : 0.0f;
+  if (j0 == 0) {
+#pragma unroll
+    for (int i = 0; i < N::NIN; i++) xs[t][i] = x[i];
+  }
   // forward
-  float a1[N::H], a2[N::H];
-#pragma unroll 4
-  for (int j = 0; j < N::H; j++) {
-    float a = P[N::oB1 + j];
+  float a1[JW], a2[JW];
 #pragma unroll
-    for (int i = 0; i < N::NIN; i++) a = fmaf(P[N::oW1 + j * N::NIN + i], x[i], a);
+  for (int j = 0; j < JW; j++) {
+    float a = P[N::oB1 + j0 + j];
+#pragma unroll
+    for (int i = 0; i < N::NIN; i++) a = fmaf(P[N::oW1 + (j0 + j) * N::NIN + i], x[i], a);
     a1[j] = a;
-    h1s[t][j] = fmaxf(a, 0.0f);
+    h1s[t][j0 + j] = fmaxf(a, 0.0f);
   }
-#pragma unroll 4
-  for (int j = 0; j < N::H; j++) {
-    float a = P[N::oB2 + j];
+  __syncthreads();
 #pragma unroll
-    for (int i = 0; i < N::H; i++) a = fmaf(P[N::oW2 + j * N::H + i], fmaxf(a1[i], 0.0f), a);
+  for (int j = 0; j < JW; j++) {
+    float a = P[N::oB2 + j0 + j];
+#pragma unroll
+    for (int i = 0; i < N::H; i++) a = fmaf(P[N::oW2 + (j0 + j) * N::H + i], h1s[t][i], a);
     a2[j] = a;
-    h2s[t][j] = fmaxf(a, 0.0f);
+    h2s[t][j0 + j] = fmaxf(a, 0.0f);
   }
+  __syncthreads();
   float z = P[N::oB3];
 #pragma unroll
-  for (int i = 0; i < N::H; i++) z = fmaf(P[N::oW3 + i], fmaxf(a2[i], 0.0f), z);
+  for (int i = 0; i < N::H; i++) z = fmaf(P[N::oW3 + i], h2s[t][i], z);
   // loss and its derivative in z
   const float w = y > 0.5f ? posW : 1.0f;
   const float m = y > 0.5f ? -z : z;  // softplus argument
   const float sp = fmaxf(m, 0.0f) + log1pf(expf(-fabsf(m)));
   const float sig = 1.0f / (1.0f + expf(-z));
   const float dz = live ? w * (sig - y) : 0.0f;
-  ls[t] = live ? w * sp : 0.0f;
-  dzs[t] = dz;
+  if (j0 == 0) {
+    ls[t] = live ? w * sp : 0.0f;
+    dzs[t] = dz;
+  }
   // backward through the hidden layers
 #pragma unroll
-  for (int j = 0; j < N::H; j++) d2s[t][j] = a2[j] > 0.0f ? dz * P[N::oW3 + j] : 0.0f;
-#pragma unroll 4
-  for (int i = 0; i < N::H; i++) {
+  for (int j = 0; j < JW; j++) d2s[t][j0 + j] = a2[j] > 0.0f ? dz * P[N::oW3 + j0 + j] : 0.0f;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < JW; i++) {
     float acc = 0.0f;
 #pragma unroll
-    for (int j = 0; j < N::H; j++) acc = fmaf(d2s[t][j], P[N::oW2 + j * N::H + i], acc);
-    d1s[t][i] = a1[i] > 0.0f ? acc : 0.0f;
+    for (int j = 0; j < N::H; j++) acc = fmaf(d2s[t][j], P[N::oW2 + j * N::H + j0 + i], acc);
+    d1s[t][j0 + i] = a1[i] > 0.0f ? acc : 0.0f;
   }
   __syncthreads();
   // parameter gradients summed over the block's samples (ascending sample order)
   float *out = part + size_t(blockIdx.x) * N::NP;
-  for (int p = t; p < N::NP; p += TB) {
+  for (int p = threadIdx.x; p < N::NP; p += TB * TW) {
     float acc = 0.0f;
     if (p < N::oB1) {
       const int j = p / N::NIN, i = p % N::NIN;
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc = fmaf(d1s[q][j], xs[q][i], acc);
     } else if (p < N::oW2) {
       const int j = p - N::oB1;
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc += d1s[q][j];
     } else if (p < N::oB2) {
       const int j = (p - N::oW2) / N::H, i = (p - N::oW2) % N::H;
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc = fmaf(d2s[q][j], h1s[q][i], acc);
     } else if (p < N::oW3) {
       const int j = p - N::oB2;
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc += d2s[q][j];
     } else if (p < N::oB3) {
       const int i = p - N::oW3;
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc = fmaf(dzs[q], h2s[q][i], acc);
     } else {
+#pragma unroll 16
       for (int q = 0; q < TB; q++) acc += dzs[q];
     }
     out[p] = acc;
   }
-  if (t == 0) {
+  if (threadIdx.x == TB * TW - 1) {
     float l = 0.0f;
+#pragma unroll 16
     for (int q = 0; q < TB; q++) l += ls[q];
     lossPart[blockIdx.x] = l;
   }
 }
 
 #ifdef KFVM_SMALL_KERNELS
-// grad[p] = sum over blocks of part[blk][p] / nb (fixed order); loss likewise.
-__global__ __launch_bounds__(BLK) void k_train_reduce(const float *__restrict__ part,
-                                                      const float *__restrict__ lossPart, int nblk,
-                                                      int np, int nb, float *__restrict__ grad,
-                                                      float *__restrict__ loss) {
-  const int p = blockIdx.x * BLK + threadIdx.x;
-  if (p < np) {
-    float acc = 0.0f;
-    for (int b = 0; b < nblk; b++) acc += part[size_t(b) * np + p];
-    grad[p] = acc / float(nb);
-  }
-  if (p == 0) {
-    float l = 0.0f;
-    for (int b = 0; b < nblk; b++) l += lossPart[b];
-    *loss = l / float(nb);
-  }
-}
-
 // bfloat16 rounding (to nearest, ties to even) of a float, kept as a float.
 __device__ inline float bf16_round(float v) {
   uint32_t u = __float_as_uint(v);
@@ -736,22 +739,46 @@ __device__ inline float bf16_round(float v) {
   return __uint_as_float(u & 0xffff0000u);
 }
 
-// Adam step on the FP32 master parameters M; Pbf receives their bfloat16
-// values, which the forward pass uses.
-__global__ __launch_bounds__(BLK) void k_adam(float *__restrict__ M, float *__restrict__ Pbf,
-                                              const float *__restrict__ grad, float *__restrict__ m1,
-                                              float *__restrict__ m2, int np, float lr, float b1,
-                                              float b2, float eps, float c1, float c2) {
-  const int p = blockIdx.x * BLK + threadIdx.x;
-  if (p >= np) return;
-  const float gp = grad[p];
-  const float a = b1 * m1[p] + (1.0f - b1) * gp;
-  const float v = b2 * m2[p] + (1.0f - b2) * gp * gp;
-  m1[p] = a;
-  m2[p] = v;
-  const float th = M[p] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-  M[p] = th;
-  Pbf[p] = bf16_round(th);
+// grad[p] = sum over blocks of part[blk][p] / nb (fixed order), the loss likewise
+// (thread np); then, with AdamArgs::M, the Adam step of that parameter on the
+// FP32 master parameters M; Pbf receives their bfloat16 values, which the
+// forward pass uses.  The partials of 32 blocks are in flight at once: one load
+// at a time left the 128 of a batch of 8192 samples a chain of 36 us, plus a
+// launch for the step; now 5 us.
+constexpr int TRB = 64;  // threads per block: few parameters, spread over the CUs
+__global__ __launch_bounds__(TRB) void k_train_reduce(const float *__restrict__ part,
+                                                     const float *__restrict__ lossPart, int nblk,
+                                                     int np, int nb, float *__restrict__ grad,
+                                                     float *__restrict__ loss, AdamArgs ad) {
+  const int p = blockIdx.x * TRB + threadIdx.x;
+  if (p > np) return;
+  const float *src = p < np ? part + p : lossPart;
+  const size_t stride = p < np ? size_t(np) : 1;
+  float acc = 0.0f;
+  constexpr int K = 32;
+  int b = 0;
+  for (; b + K <= nblk; b += K) {
+    float v[K];
+#pragma unroll
+    for (int e = 0; e < K; e++) v[e] = src[(b + e) * stride];
+#pragma unroll
+    for (int e = 0; e < K; e++) acc += v[e];
+  }
+  for (; b < nblk; b++) acc += src[b * stride];
+  const float gp = acc / float(nb);
+  if (p == np) {
+    *loss = gp;
+    return;
+  }
+  grad[p] = gp;
+  if (!ad.M) return;
+  const float a = ad.b1 * ad.m1[p] + (1.0f - ad.b1) * gp;
+  const float v = ad.b2 * ad.m2[p] + (1.0f - ad.b2) * gp * gp;
+  ad.m1[p] = a;
+  ad.m2[p] = v;
+  const float th = ad.M[p] - ad.lr * (a / ad.c1) / (sqrtf(v / ad.c2) + ad.eps);
+  ad.M[p] = th;
+  ad.Pbf[p] = bf16_round(th);
 }
 
 #endif  // KFVM_SMALL_KERNELS

@@ -292,7 +292,7 @@ template <int D, int NQ>
 hipError_t Launch<D, NQ>::train_grad(const float *X, const float *Y, const int *idx, int n, int nb, uint64_t seed,
                                      const float *P, float posW, float *part, float *lossPart, hipStream_t s) {
   const unsigned nblk = unsigned((nb + dev::TB - 1) / dev::TB);
-  hipLaunchKernelGGL((dev::k_train_grad<D>), dim3(nblk), dim3(dev::TB), 0, s, X, Y, idx, n, nb, seed, P, posW,
+  hipLaunchKernelGGL((dev::k_train_grad<D>), dim3(nblk), dim3(dev::TB * dev::TW), 0, s, X, Y, idx, n, nb, seed, P, posW,
                      part, lossPart);
   return hipGetLastError();
 }

@@ -141,7 +141,7 @@ void Indicator::getBf16(uint16_t *W) const {
 }
 
 void Indicator::gradOn(const float *dP, const float *dX, const float *dY, const int *dIdx, int64_t n, int nb,
-                       uint64_t seed, double posWeight) {
+                       uint64_t seed, double posWeight, const AdamArgs &ad) {
   const int tb = net_train_block();
   const int nblk = (nb + tb - 1) / tb;
   if (nblk > partBlocks_) {
@@ -154,7 +154,7 @@ void Indicator::gradOn(const float *dP, const float *dX, const float *dY, const 
   }
   check(launch_train_grad(dim_, dX, dY, dIdx, int(n), nb, seed, dP, float(posWeight), part_, lossPart_, stream_),
         "train_grad");
-  check(launch_train_reduce(part_, lossPart_, nblk, np_, nb, grad_, loss_, stream_), "train_reduce");
+  check(launch_train_reduce(part_, lossPart_, nblk, np_, nb, grad_, loss_, ad, stream_), "train_reduce");
 }
 
 double Indicator::train(int iters, int batch, double lr, double posWeight, uint64_t seed) {
@@ -163,10 +163,10 @@ double Indicator::train(int iters, int batch, double lr, double posWeight, uint6
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int it = 0; it < iters; it++) {
     step_++;
-    gradOn(Pbf_, X_, Y_, nullptr, n_, batch, splitmix(seed + uint64_t(step_)), posWeight);
     const float c1 = float(1.0 - std::pow(double(b1), double(step_)));
     const float c2 = float(1.0 - std::pow(double(b2), double(step_)));
-    check(launch_adam(M_, Pbf_, grad_, m1_, m2_, np_, float(lr), b1, b2, eps, c1, c2, stream_), "adam");
+    gradOn(Pbf_, X_, Y_, nullptr, n_, batch, splitmix(seed + uint64_t(step_)), posWeight,
+           AdamArgs{M_, Pbf_, m1_, m2_, float(lr), b1, b2, eps, c1, c2});
   }
   float l = 0.0f;
   check(hipMemcpyAsync(&l, loss_, sizeof(float), hipMemcpyDeviceToHost, stream_), "loss");
@@ -188,7 +188,7 @@ double Indicator::gradient(const float *P, const float *X, const float *Y, int64
     check(hipMemcpy(dX, X, size_t(n) * nin_ * sizeof(float), hipMemcpyHostToDevice), "X");
     check(hipMemcpy(dY, Y, size_t(n) * sizeof(float), hipMemcpyHostToDevice), "Y");
     check(hipMemcpy(dIdx, idx.data(), size_t(n) * sizeof(int), hipMemcpyHostToDevice), "idx");
-    gradOn(dP, dX, dY, dIdx, n, int(n), 0, posWeight);
+    gradOn(dP, dX, dY, dIdx, n, int(n), 0, posWeight, AdamArgs{});
     float lf = 0.0f;
     check(hipMemcpyAsync(grad, grad_, size_t(np_) * sizeof(float), hipMemcpyDeviceToHost, stream_), "grad");
     check(hipMemcpyAsync(&lf, loss_, sizeof(float), hipMemcpyDeviceToHost, stream_), "loss");

@@ -9,6 +9,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "../device/device_api.hpp"
+
 namespace kfvm {
 
 class Solver;
@@ -48,7 +50,7 @@ class Indicator {
  private:
   void reserve(int64_t n);
   void gradOn(const float *dP, const float *dX, const float *dY, const int *dIdx, int64_t n, int nb,
-              uint64_t seed, double posWeight);
+              uint64_t seed, double posWeight, const AdamArgs &ad);
 
   int dim_, nin_, np_;
   int64_t n_ = 0, cap_ = 0, npos_ = 0;
