@@ -227,13 +227,9 @@ hipError_t LaunchMhd<D, NQ>::weno(const double *U, double *FS, double *SRC, cons
   else
     hipLaunchKernelGGL((dev::k_mhd_wenorec<D, NQ>), dim3(nb), dim3(dev::BLK), 0, s, U, FS, SRC, g, FT, DT, CT,
                        list, counter, WC);
-  const unsigned np = std::min<unsigned>(stage_blocks(g.ncell), 1u << 16);
-  if (list)
-    hipLaunchKernelGGL((dev::k_mhd_weno_post<D, NQ>), dim3(np), dim3(dev::BLK), 0, s, U, FS, SRC, g, list,
-                       counter, thetaNew, spd, props);
-  else
-    hipLaunchKernelGGL((dev::k_mhd_weno_post_cells<D, NQ>), dim3(np), dim3(dev::BLK), 0, s, U, FS, SRC, g,
-                       thetaNew, spd, props);
+  const unsigned np = std::min<unsigned>((unsigned(g.ncell) + 63) / 64, 1u << 14);
+  hipLaunchKernelGGL((dev::k_mhd_weno_post<D, NQ>), dim3(np), dim3(64), 0, s, U, FS, SRC, g, list, counter, thetaNew,
+                     spd, props);
   return hipGetLastError();
 }
 
