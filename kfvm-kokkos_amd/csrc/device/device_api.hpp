@@ -7,6 +7,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <cstdlib>
 
 namespace kfvm {
 
@@ -193,6 +194,8 @@ hipError_t launch_select(int dim, int nq, const double *U, const double *WI, con
 // WP (may be null; also launch_mhd_weno's): the mirror-symmetric form of the
 // weights (host/parity_weno.hpp), which then takes the place of the dense
 // tables; the grid must have fewer than 2^29 cells (32-bit byte offsets).
+// props (may be null; needs WP, a list with a row for every cell, a shape of
+// fused_flux and !weno_scalar()): launch_weno_post's work is done as well.
 // Compact WENO weight table (see launch_weno) from the reference layouts
 // face [nSub][F*Q][C] and deriv [nSub][I][C]; out has SUB*(F*Q + I) doubles,
 // then, with nCell > 0 (GLM-MHD), SUB*nCell rows of the interior-point
@@ -202,7 +205,13 @@ void compact_weno_weights(int dim, int fq, int nI, const double *face, const dou
 hipError_t launch_weno(int dim, int nq, int nv, const double *U, double *FS, double *thetaNew,
                        const Grid &g, const double *FW, const double *DW, const double *FWS,
                        const double *DWS, const int *list, const int *counter, double *WS, int cap,
-                       const double *WP, hipStream_t s);
+                       const double *WP, const double *props, hipStream_t s);
+// KFVM_WENO_SCALAR=1 (read at every launch) runs the Euler WENO on the scalar
+// kernel: the others are compared with it in the tests.
+inline bool weno_scalar() {
+  const char *ev = std::getenv("KFVM_WENO_SCALAR");
+  return ev && ev[0] == '1';
+}
 // Euler: back to conserved variables and the positivity limiter on the
 // listed cells (in WS for the first cap of them, then copied to FS).
 hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double *thetaNew,

@@ -81,11 +81,11 @@ void compact_weno_weights(int dim, int fq, int nI, const double *face, const dou
 hipError_t launch_weno(int dim, int nq, int nv, const double *U, double *FS, double *thetaNew,
                        const Grid &g, const double *FW, const double *DW, const double *FWS,
                        const double *DWS, const int *list, const int *counter, double *WS, int cap,
-                       const double *WP, hipStream_t s) {
+                       const double *WP, const double *props, hipStream_t s) {
   if (nv != 5 && nv != 1) return hipErrorInvalidValue;
   if (WS && cap < 0) return hipErrorInvalidValue;
   (void)DWS;
-  KFVM_SELECT(dim, nq, L::weno(nv, U, FS, thetaNew, g, FW, DW, list, counter, WS, cap, nv == 5 ? FWS : nullptr, WP, s));
+  KFVM_SELECT(dim, nq, L::weno(nv, U, FS, thetaNew, g, FW, DW, list, counter, WS, cap, nv == 5 ? FWS : nullptr, WP, props, s));
 }
 
 hipError_t launch_weno_post(int dim, int nq, const double *U, double *FS, double *thetaNew,

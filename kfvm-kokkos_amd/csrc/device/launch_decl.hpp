@@ -25,7 +25,8 @@ struct Launch {
                            hipStream_t s);
   static hipError_t weno(int nv, const double *U, double *FS, double *thetaNew, const Grid &g,
                          const double *FW, const double *DW, const int *list, const int *counter,
-                         double *WS, int cap, const double *WC, const double *WP, hipStream_t s);
+                         double *WS, int cap, const double *WC, const double *WP, const double *props,
+                         hipStream_t s);
   // ---- fused path (Euler, sparse WENO)
   static hipError_t linear_surf(const double *U, double *WI, double *thetaNew, const double *props,
                                 const Grid &g, const double *PW, int *ppList, int *ppCount, double *SB,

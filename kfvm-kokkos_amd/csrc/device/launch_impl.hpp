@@ -65,16 +65,24 @@ hipError_t Launch<D, NQ>::select(const double *U, const double *WI, const double
 template <int D, int NQ>
 hipError_t Launch<D, NQ>::weno(int nv, const double *U, double *FS, double *thetaNew, const Grid &g,
                                const double *FW, const double *DW, const int *list, const int *counter,
-                               double *WS, int cap, const double *WC, const double *WP, hipStream_t s) {
+                               double *WS, int cap, const double *WC, const double *WP, const double *props,
+                               hipStream_t s) {
   if (nv == 5) {
-    // KFVM_WENO_SCALAR=1 (read at every launch) runs the scalar kernel
-    // instead: the others are compared with it in the tests
-    const char *ev = std::getenv("KFVM_WENO_SCALAR");
-    const bool scalar = ev && ev[0] == '1';
+    const bool scalar = weno_scalar();
     if (WP && !scalar) {
       using K = dev::WenoPar<D, NQ, 5>;
-      hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 5>), dim3(weno_par_blocks(g)), dim3(K::NT), 0, s, U, FS, nullptr, g,
-                         WP, list, counter, WS, WS ? cap : 0);
+      const dim3 nb(weno_par_blocks(g)), nt(K::NT);
+      if constexpr (fused_flux(D, NQ)) {
+        if (props) {
+          if (!list || !WS || cap < g.ncell) return hipErrorInvalidValue;
+          hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 5, true>), nb, nt, 0, s, U, FS, nullptr, g, WP, list, counter,
+                             WS, cap, thetaNew, props);
+          return hipGetLastError();
+        }
+      }
+      if (props) return hipErrorInvalidValue;
+      hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 5, false>), nb, nt, 0, s, U, FS, nullptr, g, WP, list, counter, WS,
+                         WS ? cap : 0, nullptr, nullptr);
       return hipGetLastError();
     }
     // persistent: every workgroup stages the weights once, then strides over the list
@@ -222,8 +230,9 @@ hipError_t LaunchMhd<D, NQ>::weno(const double *U, double *FS, double *SRC, cons
   if (lds && !WC) return hipErrorInvalidValue;
   const unsigned nb = std::min<unsigned>(unsigned((g.ncell + dev::MCPB - 1) / dev::MCPB), lds ? 2048u : 1u << 16);
   if (WP)
-    hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 9>), dim3(weno_par_blocks(g)), dim3(dev::WenoPar<D, NQ, 9>::NT), 0, s,
-                       U, FS, SRC, g, WP, list, counter, nullptr, 0);
+    hipLaunchKernelGGL((dev::k_weno_par<D, NQ, 9, false>), dim3(weno_par_blocks(g)),
+                       dim3(dev::WenoPar<D, NQ, 9>::NT), 0, s, U, FS, SRC, g, WP, list, counter, nullptr, 0, nullptr,
+                       nullptr);
   else
     hipLaunchKernelGGL((dev::k_mhd_wenorec<D, NQ>), dim3(nb), dim3(dev::BLK), 0, s, U, FS, SRC, g, FT, DT, CT,
                        list, counter, WC);

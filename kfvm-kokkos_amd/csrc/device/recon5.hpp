@@ -976,8 +976,67 @@ __device__ inline PPBounds pp_bounds_p(const double *__restrict__ U,
 template <int FQ>
 struct PostGroup {
   static constexpr int G = FQ <= 24 ? 8 : 16;
-  static constexpr int PPL = (FQ + G - 1) / G;  // points per lane
 };
+
+// The pass on one cell by a group of G lanes (lane pl of it): state w of point
+// pt at P[(pt * 5 + w) * ps].  Returns the cell's theta.
+template <int D, int NQ, int G>
+__device__ __forceinline__ double weno_post_cell(double *P, size_t ps, const double *__restrict__ U,
+                                                 const double *__restrict__ props, const Grid &g, int c, int pl) {
+  constexpr int FQ = Shape<D, NQ>::F * Shape<D, NQ>::Q, PPL = (FQ + G - 1) / G;
+  const size_t nc = g.ncell;
+  int i, j, k;
+  cell_ijk<D>(c, g, i, j, k);
+  double ref[5];
+#pragma unroll
+  for (int w = 0; w < 5; w++) ref[w] = U[size_t(w) * nc + c];
+  const PPBounds pb = grp_pp_bounds<D, G>(U, props, g, i, j, k, ref, pl);
+  const LinPrim lp(ref, g.gamma);
+  const double ru = lp.rho * lp.u, rvv = lp.rho * lp.v, rw = lp.rho * lp.w;
+  double st[PPL][5];
+  double thDl = 1.0;
+#pragma unroll
+  for (int e = 0; e < PPL; e++) {
+    const int pt = pl + G * e;
+    if (pt < FQ) {
+      const double *q = P + size_t(pt * 5) * ps;
+      const double d = q[0], mx = q[ps], my = q[2 * ps], mz = q[3 * ps], en = q[4 * ps];
+      st[e][4] = (lp.vsq * d + ru * mx + rvv * my + rw * mz + en / lp.gamm);
+      st[e][1] = (lp.rho * mx + lp.u * d);
+      st[e][2] = (lp.rho * my + lp.v * d);
+      st[e][3] = (lp.rho * mz + lp.w * d);
+      st[e][0] = d;
+      thDl = fmin(thDl, dens_theta(1.0, d, pb));
+    } else {
+#pragma unroll
+      for (int w = 0; w < 5; w++) st[e][w] = ref[w];
+    }
+  }
+  const double thD = grp_min<G>(thDl);
+  const bool mixD = thD > 0.0 && thD < 1.0, repD = !mixD && thD < 1.0;
+  double thEl = 1.0;
+#pragma unroll
+  for (int e = 0; e < PPL; e++) {
+#pragma unroll
+    for (int w = 0; w < 5; w++)
+      st[e][w] = repD ? ref[w] : (mixD ? ref[w] + thD * (st[e][w] - ref[w]) : st[e][w]);
+    if (pl + G * e < FQ && !(Hydro::eint(st[e]) > pb.minEint))
+      thEl = fmin(thEl, eint_pos(pb.minEint, ref, st[e]));
+  }
+  const double thP = grp_min<G>(thEl);
+  const bool mixP = thP > 0.0 && thP < 1.0, repP = !mixP && thP < 1.0;
+#pragma unroll
+  for (int e = 0; e < PPL; e++) {
+    const int pt = pl + G * e;
+    if (pt < FQ) {
+      double *const q = P + size_t(pt * 5) * ps;
+#pragma unroll
+      for (int w = 0; w < 5; w++)
+        q[w * ps] = repP ? ref[w] : (mixP ? ref[w] + thP * (st[e][w] - ref[w]) : st[e][w]);
+    }
+  }
+  return fmin(thD, thP);
+}
 
 template <int D, int NQ>
 __global__ __launch_bounds__(BLK) void k_weno_post(const double *__restrict__ U,
@@ -988,76 +1047,17 @@ __global__ __launch_bounds__(BLK) void k_weno_post(const double *__restrict__ U,
                                                    const int *__restrict__ counter,
                                                    double *__restrict__ WS, int cap) {
   constexpr int FQ = Shape<D, NQ>::F * Shape<D, NQ>::Q;
-  constexpr int G = PostGroup<FQ>::G, PPL = PostGroup<FQ>::PPL, GPW = 64 / G;
+  constexpr int G = PostGroup<FQ>::G, GPW = 64 / G;
   const int n = list ? *counter : g.ncell;
   const int lane = threadIdx.x & 63, pl = lane % G;
   const int gid = (blockIdx.x * (BLK / 64) + (threadIdx.x >> 6)) * GPW + lane / G;
   const int ngroups = gridDim.x * (BLK / 64) * GPW;
-  const size_t nc = g.ncell;
   for (int t = gid; t < n; t += ngroups) {
     const int c = list ? list[t] : t;
     const bool compact = list && t < cap;
-    int i, j, k;
-    cell_ijk<D>(c, g, i, j, k);
-    double ref[5];
-#pragma unroll
-    for (int w = 0; w < 5; w++) ref[w] = U[size_t(w) * nc + c];
-    const PPBounds pb = grp_pp_bounds<D, G>(U, props, g, i, j, k, ref, pl);
-    const LinPrim lp(ref, g.gamma);
-    const double ru = lp.rho * lp.u, rvv = lp.rho * lp.v, rw = lp.rho * lp.w;
-    double st[PPL][5];
-    double thDl = 1.0;
-#pragma unroll
-    for (int e = 0; e < PPL; e++) {
-      const int pt = pl + G * e;
-      if (pt < FQ) {
-        double a[5];
-        if (compact) {
-          const double *q = WS + size_t(t) * (FQ * 5) + pt * 5;
-#pragma unroll
-          for (int w = 0; w < 5; w++) a[w] = q[w];
-        } else {
-          const double *q = FS + fs_base(c, FQ * 5) + (size_t(pt) * 5) * FSB;
-#pragma unroll
-          for (int w = 0; w < 5; w++) a[w] = q[w * FSB];
-        }
-        const double d = a[0], mx = a[1], my = a[2], mz = a[3], en = a[4];
-        st[e][4] = (lp.vsq * d + ru * mx + rvv * my + rw * mz + en / lp.gamm);
-        st[e][1] = (lp.rho * mx + lp.u * d);
-        st[e][2] = (lp.rho * my + lp.v * d);
-        st[e][3] = (lp.rho * mz + lp.w * d);
-        st[e][0] = d;
-        thDl = fmin(thDl, dens_theta(1.0, d, pb));
-      } else {
-#pragma unroll
-        for (int w = 0; w < 5; w++) st[e][w] = ref[w];
-      }
-    }
-    const double thD = grp_min<G>(thDl);
-    const bool mixD = thD > 0.0 && thD < 1.0, repD = !mixD && thD < 1.0;
-    double thEl = 1.0;
-#pragma unroll
-    for (int e = 0; e < PPL; e++) {
-#pragma unroll
-      for (int w = 0; w < 5; w++)
-        st[e][w] = repD ? ref[w] : (mixD ? ref[w] + thD * (st[e][w] - ref[w]) : st[e][w]);
-      if (pl + G * e < FQ && !(Hydro::eint(st[e]) > pb.minEint))
-        thEl = fmin(thEl, eint_pos(pb.minEint, ref, st[e]));
-    }
-    const double thP = grp_min<G>(thEl);
-    const bool mixP = thP > 0.0 && thP < 1.0, repP = !mixP && thP < 1.0;
-#pragma unroll
-    for (int e = 0; e < PPL; e++) {
-      const int pt = pl + G * e;
-      if (pt < FQ) {
-        double *const q = compact ? WS + size_t(t) * (FQ * 5) + pt * 5 : FS + fs_base(c, FQ * 5) + (size_t(pt) * 5) * FSB;
-        const size_t qs = compact ? 1 : FSB;
-#pragma unroll
-        for (int w = 0; w < 5; w++)
-          q[w * qs] = repP ? ref[w] : (mixP ? ref[w] + thP * (st[e][w] - ref[w]) : st[e][w]);
-      }
-    }
-    if (pl == 0) thetaNew[c] = fmin(thD, thP);
+    double *const P = compact ? WS + size_t(t) * (FQ * 5) : FS + fs_base(c, FQ * 5);
+    const double th = weno_post_cell<D, NQ, G>(P, compact ? 1 : FSB, U, props, g, c, pl);
+    if (pl == 0) thetaNew[c] = th;
   }
 }
 

@@ -274,21 +274,30 @@ struct WenoPar {
   static constexpr int NT = 64 * NV;
   static constexpr int ROW = N * NV + 1;  // LDS row of one cell and face axis, padded against bank conflicts
   static constexpr int VALS = (NV - 1) * SInfo<D>::C * 64;  // stencil values of all variables but the energy
-  static constexpr int LDS = NV == 5 && 64 * ROW > VALS ? 64 * ROW : VALS;
+  // POST: whole rows of the cells in LDS, then lanes per cell for the limiter
+  static constexpr int ROWF = FQ * NV + 1, G = 4;
+  static constexpr int lds(bool post) {
+    const int r = NV != 5 ? 0 : 64 * (post ? ROWF : ROW);
+    return r > VALS ? r : VALS;
+  }
   // 3D 3x3: 18 accumulators and their points need the 256 registers of two waves per SIMD
   static constexpr int WAVES = D == 3 && NQ == 3 ? 2 : 3;
 };
 
-template <int D, int NQ, int NV>
+// POST (Euler, every listed cell has a row): the workgroup also does k_weno_post's
+// work on its cells while their rows are in LDS, so that they cross HBM once:
+// 160 x 144 x 152 0.68 ms for both instead of 0.46 + 0.30, 64^3 87 us instead of
+// 62 + 29 and a launch.
+template <int D, int NQ, int NV, bool POST>
 __global__ __launch_bounds__((WenoPar<D, NQ, NV>::NT), (WenoPar<D, NQ, NV>::WAVES)) void k_weno_par(
     const double *__restrict__ U, double *__restrict__ FS, double *__restrict__ SRC, Grid g,
     const double *__restrict__ WP, const int *__restrict__ list, const int *__restrict__ counter,
-    double *__restrict__ WS, int cap) {
+    double *__restrict__ WS, int cap, double *__restrict__ thetaNew, const double *__restrict__ props) {
   using K = WenoPar<D, NQ, NV>;
   constexpr int C = SInfo<D>::C, nSub = SInfo<D>::nSub, N = K::N, FQ = K::FQ;
   constexpr double gHi = 0.7, gLo = 0.7;
   constexpr double g0 = gHi, g1 = (1.0 - gHi) * gLo, gb = (1.0 - gHi) * (1.0 - gLo) / double(2 * D);
-  __shared__ double lds[K::LDS];
+  __shared__ double lds[K::lds(POST)];
   const int n = list ? *counter : g.ncell;
   const int lane = threadIdx.x & 63;
   const int v = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
@@ -364,7 +373,11 @@ __global__ __launch_bounds__((WenoPar<D, NQ, NV>::NT), (WenoPar<D, NQ, NV>::WAVE
       double out[N];
       weno_points<D, NQ, A>(t, WP, om, out);
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (NV == 5) {
+      if constexpr (POST) {
+        if (A == 0) __syncthreads();  // what the rows overwrite has been read
+#pragma unroll
+        for (int p = 0; p < N; p++) lds[lane * K::ROWF + (A * N + p) * NV + v] = out[p];
+      } else if constexpr (NV == 5) {
         if (list) {
           __syncthreads();  // what the rows overwrite has been read
 #pragma unroll
@@ -387,6 +400,19 @@ __global__ __launch_bounds__((WenoPar<D, NQ, NV>::NT), (WenoPar<D, NQ, NV>::WAVE
         for (int p = 0; p < N; p++) d[size_t(p * NV) * FSB] = out[p];
       }
     });
+    if constexpr (POST) {
+      __syncthreads();
+      const int m = threadIdx.x / K::G;
+      if (m < 64 && t0 + m < n) {  // whole groups of lanes
+        const int cell = list[t0 + m], pl = threadIdx.x % K::G;
+        const double th = weno_post_cell<D, NQ, K::G>(lds + m * K::ROWF, 1, U, props, g, cell, pl);
+        if (pl == 0) thetaNew[cell] = th;
+      }
+      __syncthreads();
+      const int rows = n - t0 < 64 ? n - t0 : 64;
+      for (int x = threadIdx.x; x < rows * FQ * NV; x += K::NT)
+        WS[size_t(t0) * (FQ * NV) + x] = lds[x / (FQ * NV) * K::ROWF + x % (FQ * NV)];
+    }
     if constexpr (NV == 9) {
       constexpr int NI = ParPts<D, NQ, -1>::N;
       double out[NI];

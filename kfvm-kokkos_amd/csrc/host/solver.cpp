@@ -771,13 +771,16 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
         return launch_select(dim, nq, Uin, WI_, thPrev, wflag_, list_, counter_, wThresh, grid_, pos_, cap,
                              stream_);
       });
+    // the mirror-symmetric kernel limits the rows while it has them
+    const double *wp = weno_scalar() ? nullptr : wenoWeights(true);
     timed("weno", [&] {
       return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_, counter_,
-                         FS_, cap, wenoWeights(true), stream_);
+                         FS_, cap, wp, wp ? props_ : nullptr, stream_);
     });
-    timed("weno_post", [&] {
-      return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, FS_, cap, stream_);
-    });
+    if (!wp)
+      timed("weno_post", [&] {
+        return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, FS_, cap, stream_);
+      });
     timed("pp", [&] {
       return launch_pp_rows(dim, nq, Uin, FS_, pos_, thNew, props_, wflag_, grid_, parW_, ppList_, counter_ + 1,
                             counter_, counter_ + 2, stream_);
@@ -803,7 +806,7 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
         });
       timed("weno", [&] {
         return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, list_,
-                           counter_, WS_, cap, wenoWeights(true), stream_);
+                           counter_, WS_, cap, wenoWeights(true), nullptr, stream_);
       });
       timed("weno_post", [&] {
         return launch_weno_post(dim, nq, Uin, FS_, thNew, props_, grid_, list_, counter_, WS_, cap, stream_);
@@ -815,7 +818,7 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   } else {
     timed("weno", [&] {
       return launch_weno(dim, nq, nv_, Uin, FS_, thNew, grid_, faceW_, derivW_, faceWC_, derivWS_, nullptr,
-                         nullptr, nullptr, 0, wenoWeights(false), stream_);
+                         nullptr, nullptr, 0, wenoWeights(false), nullptr, stream_);
     });
     if (hydro)
       timed("weno_post", [&] {
@@ -1158,7 +1161,7 @@ void Solver::collectSamples(float *X, float *Y, double tau) {
         "linear");
   check(hipMemcpyAsync(FSlin_, FS_, fsBytes, hipMemcpyDeviceToDevice, stream_), "copy linear states");
   check(launch_weno(dim, nq, nv_, Uin, FS_, thScratch, grid_, faceW_, derivW_, faceWC_, derivWS_, nullptr, nullptr,
-                    nullptr, 0, wenoWeights(false), stream_),
+                    nullptr, 0, wenoWeights(false), nullptr, stream_),
         "weno");
   check(launch_weno_post(dim, nq, Uin, FS_, thScratch, props_, grid_, nullptr, nullptr, nullptr, 0, stream_),
         "weno_post");
