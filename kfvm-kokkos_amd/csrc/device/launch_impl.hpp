@@ -34,10 +34,15 @@ hipError_t Launch<D, NQ>::linear(int nv, const double *U, double *FS, double *WI
                                  const double *props, const Grid &g, const double *W0, const double *W0T,
                                  int *ppList, int *ppCount, hipStream_t s, const LearnArgs *la, const double *PW) {
   const dim3 nb(bricks(g)), nt(dev::RBox<D>::NT);
-  if (nv == 5 && PW && la)
-    hipLaunchKernelGGL((dev::k_linear_par<D, NQ, false, true>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, PW,
-                       ppList, ppCount, nullptr, Surf{}, *la);
-  else if (nv == 5 && PW)
+  if constexpr (D == 2) {
+    if (nv == 5 && PW && la) {
+      hipLaunchKernelGGL((dev::k_linear_par<D, NQ, false, true>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, PW,
+                         ppList, ppCount, nullptr, Surf{}, *la);
+      return hipGetLastError();
+    }
+  }
+  if (PW && la) return hipErrorInvalidValue;  // the learned selection in 3D keeps the dense pass
+  if (nv == 5 && PW)
     hipLaunchKernelGGL((dev::k_linear_par<D, NQ, false, false>), nb, nt, 0, s, U, FS, WI, thetaNew, props, g, PW,
                        ppList, ppCount, nullptr, Surf{}, LearnArgs{});
   else if (nv == 5 && la)
@@ -112,12 +117,16 @@ hipError_t Launch<D, NQ>::linear_surf(const double *U, double *WI, double *theta
                                       const Surf &sb, hipStream_t s, const LearnArgs *la) {
   if constexpr (fused_flux(D, NQ)) {
     const dim3 nb(bricks(g)), nt(dev::RBox<D>::NT);
-    if (la)
-      hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, true>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g,
-                         PW, ppList, ppCount, SB, sb, *la);
-    else
-      hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, false>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g,
-                         PW, ppList, ppCount, SB, sb, LearnArgs{});
+    if constexpr (D == 2) {
+      if (la) {
+        hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, true>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g,
+                           PW, ppList, ppCount, SB, sb, *la);
+        return hipGetLastError();
+      }
+    }
+    if (la) return hipErrorInvalidValue;  // the learned selection in 3D keeps the dense pass
+    hipLaunchKernelGGL((dev::k_linear_par<D, NQ, true, false>), nb, nt, 0, s, U, nullptr, WI, thetaNew, props, g, PW,
+                       ppList, ppCount, SB, sb, LearnArgs{});
     return hipGetLastError();
   } else {
     return hipErrorInvalidValue;
