@@ -203,8 +203,11 @@ __global__ __launch_bounds__(RBox<D>::NT, D == 3 && NQ == 3 ? 2 : 3) void k_line
     // Fast test of the limiter: every density strictly inside the bounds and
     // every internal energy above its bound by more than rounding, without the
     // exact sequence's divisions.  A cell that fails, or only touches a bound,
-    // goes to the exact sequence, which then decides.
-    bool ok = true;
+    // goes to the exact sequence, which then decides.  The tests are formed where
+    // their values are (keep_here): as a chain of conditions they were put off to
+    // the end, with the values (3x3 rule: 256 registers and scratch, now 200;
+    // 75 x 62 x 81 0.395 -> 0.367 ms, 2D 1024^2 0.099 -> 0.090).
+    int bad = 0;
     static_for<D / AXG>([&](auto grp) KFVM_INLINE {
       constexpr int A0 = decltype(grp)::value * AXG;
       double rho[AXG * 2 * Q], msq[AXG * 2 * Q];
@@ -243,16 +246,21 @@ __global__ __launch_bounds__(RBox<D>::NT, D == 3 && NQ == 3 ? 2 : 3) void k_line
 #pragma unroll
             for (int p = 0; p < 2 * Q; p++) {
               rho[P0 + p] = out[p];
-              ok = ok && out[p] > pb.minDens && out[p] < pb.maxDens && out[p] > 0.0;
+              bad |= !((out[p] > pb.minDens) & (out[p] < pb.maxDens) & (out[p] > 0.0));
+              keep_here(bad);
             }
           } else if constexpr (v < 4) {
 #pragma unroll
-            for (int p = 0; p < 2 * Q; p++) msq[P0 + p] = v == 1 ? out[p] * out[p] : msq[P0 + p] + out[p] * out[p];
+            for (int p = 0; p < 2 * Q; p++) {
+              msq[P0 + p] = v == 1 ? out[p] * out[p] : msq[P0 + p] + out[p] * out[p];
+              keep_here(msq[P0 + p]);
+            }
           } else {
 #pragma unroll
             for (int p = 0; p < 2 * Q; p++) {
               const double lhs = (out[p] - 1e-14 * fabs(out[p]) - pb.minEint) * rho[P0 + p];
-              ok = ok && lhs > 0.5 * msq[P0 + p];
+              bad |= !(lhs > 0.5 * msq[P0 + p]);
+              keep_here(bad);
               if constexpr (!LEARN) msq[P0 + p] = out[p] - div_n(0.5 * msq[P0 + p], rho[P0 + p]);  // eint
             }
           }
@@ -280,8 +288,8 @@ __global__ __launch_bounds__(RBox<D>::NT, D == 3 && NQ == 3 ? 2 : 3) void k_line
     });
     // Cells whose states violate a bound go to a list for the limiter's exact
     // sequence (keeping it out of this kernel keeps its waves convergent).
-    if (ok) thetaNew[cell] = 1.0;
-    append_cells(!ok, cell, ppList, ppCount);
+    if (!bad) thetaNew[cell] = 1.0;
+    append_cells(bad != 0, cell, ppList, ppCount);
   }
   // every thread of the block, live or not, runs the selection (barriers, MFMA)
   if (LEARN) learned_tail<D>(lds, la, g, i0, j0, k0, tid);
