@@ -323,6 +323,8 @@ void Solver::sliceTimes(double *t, double *dtOut) const {
 // or the learned network), so one graph is captured
 // per such key on its first use and replayed afterwards, with the host-side
 // state (parities, mode, counters) advanced as the captured run advanced it.
+// They also depend on the form of the weight tables, which chooses the kernels:
+// setWeights drops the graphs.
 // KFVM_GRAPH=0, event timing or a failed capture run the attempt eagerly.
 template <class F>
 void Solver::runAttempt(bool prime, F &&body) {
@@ -604,9 +606,7 @@ void Solver::release() noexcept {
   void *bufs[] = {SRC_, cellW_, cellWS_, diffM_, chBits_, U_[0], U_[1], Uprev_, Uhat_, K_, Utmp_, FS_, WI_, props_, theta_[0], theta_[1], wflag_, list_, counter_, ppList_,
                   faceW_, derivW_, faceWT_, faceWS_, derivWS_, errPart_, posPart_, vmax_, netP_, nadCount_, FSlin_, nadFlag_, sDtDev_, sRed_, sMask_, WS_, pos_, SB_, parW_, wenoP_, thBak_, wfBak_, faceWC_, spd_, mhdWT_, statsPart_};
   if (stream_) (void)hipStreamSynchronize(stream_);
-  for (auto &kv : graphs_)
-    if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
-  graphs_.clear();
+  dropGraphs();
   for (void *p : bufs)
     if (p) (void)hipFree(p);
   if (hostRed_) (void)hipHostFree(hostRed_);
@@ -614,6 +614,12 @@ void Solver::release() noexcept {
   if (sHost_) (void)hipHostFree(sHost_);
   if (sMaskHost_) (void)hipHostFree(sMaskHost_);
   if (stream_) (void)hipStreamDestroy(stream_);
+}
+
+void Solver::dropGraphs() noexcept {
+  for (auto &kv : graphs_)
+    if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
+  graphs_.clear();
 }
 
 template <class F>
@@ -1358,6 +1364,7 @@ void Solver::setWeights(const double *face, const double *deriv) {
   std::copy(face, face + wts_.face.size(), wts_.face.begin());
   std::copy(deriv, deriv + wts_.deriv.size(), wts_.deriv.begin());
   check(hipStreamSynchronize(stream_), "sync");
+  dropGraphs();  // captured with the kernels of the old tables' form
   uploadWeights();
 }
 // Device copies of the weight tables: the reference layouts

@@ -231,6 +231,7 @@ class Solver {
   };
   std::map<int, AttemptGraph> graphs_;
   bool graphsOn_ = false;
+  void dropGraphs() noexcept;  // after a sync of the stream
   template <class F>
   void runAttempt(bool prime, F &&body);
 

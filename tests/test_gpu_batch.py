@@ -159,6 +159,42 @@ def test_graph_replayed_steps_equal_eager_steps(kind, monkeypatch, capfd):
     assert "graph capture" not in capfd.readouterr().err
 
 
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_weights_set_between_replayed_steps(symmetric, monkeypatch):
+    """Tables set after the first steps of a batch take effect in the replayed
+    steps as in eager ones, bit for bit, whether the new tables are mirror-
+    symmetric (the kernels stay) or not (the dense kernels take over)."""
+    import kfvm_amd
+    c = config(dim=2, n=(40, 36, 1), problem="quadrant2d", user=(), fixeddt=0.002)
+    seeds = [2, 4, 6]
+    runs = {}
+    for graph in ("0", "1"):
+        monkeypatch.setenv("KFVM_GRAPH", graph)
+        runs[graph] = kfvm_amd.Solver(init_text=init_text(c), seeds=seeds)
+    # another length scale's tables, or one weight of a row moved to its neighbour
+    f, d = runs["0"].weights
+    if symmetric:
+        f, d = kfvm_amd.build_weights(2, 2, 3.0, 1.0 / 40, 1.0 / 36)
+    else:
+        f = f.copy()
+        f[0, 0, 0, :2] += np.array([1e-3, -1e-3])
+    for s in runs.values():
+        for _ in range(4):
+            assert s.take_step() == 0
+        s.set_weights(f, d)
+        for _ in range(4):
+            assert s.take_step() == 0
+    diff = np.abs(runs["1"].state - runs["0"].state).max()
+    print(f"[batch] weights set between steps, symmetric {symmetric}: replayed vs eager {diff:.3e}", flush=True)
+    assert diff == 0.0
+    assert np.array_equal(runs["1"].flags, runs["0"].flags)
+    # the new tables change the solution by more than rounding
+    old = kfvm_amd.Solver(init_text=init_text(c), seeds=seeds)
+    for _ in range(8):
+        old.take_step()
+    assert np.abs(old.state - runs["0"].state).max() > 1e-9
+
+
 @pytest.mark.parametrize("case", ["euler_batch_nq2", "mhd_nq3", "linadv"])
 def test_flux_brick_shapes_give_identical_states(case):
     """The 2D flux kernel's brick shapes (tune:fluxbrick 0 = 16x16, 1 = 32x8,
