@@ -737,6 +737,8 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   // theta of the previous RHS evaluation feeds the selector; this one writes the other buffer
   const double *thPrev = theta_[th_];
   double *thNew = theta_[th_ ^ 1];
+  const bool fused = fusedNow();
+  if (hydro && !(fused ? SB_ : WS_)) throw std::runtime_error("no device memory for the buffers of this selection");
   // counter_: [0] WENO cells, [1] cells of the linear pass for the limiter's
   // exact sequence (ppList_)
   if (hydro)  // clears the counters
@@ -745,7 +747,6 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   // the learned selection does not read the KXRCF indicator; for the Euler
   // equations it runs inside the linear pass, on the brick that pass stages
   const bool lrn = useSparseWeno && learned_ && !forcePlain_ && hydro;
-  const bool fused = fusedNow();
   const int cap = fused ? int(ncell_) : wsCap_;  // list positions with a row
   const double *PW = sym_ && !pointOrder() ? parW_ : nullptr;
   double *wi = lrn ? nullptr : WI_;
@@ -1122,6 +1123,7 @@ void Solver::setIndicator(const float *params, int np, double threshold) {
   if (slices_ > 1 && np != 0) throw std::runtime_error("the learned indicator runs on single problems");
   if (np == 0) {
     learned_ = false;
+    pathBuffers();
     return;
   }
   if (nv_ != 5 && nv_ != 9)
@@ -1445,13 +1447,20 @@ void Solver::uploadWeights() {
     check(hipMemcpy(mhdWT_, mw.data(), mw.size() * sizeof(double), hipMemcpyHostToDevice), "copy weights");
   }
 }
-// Buffers of the sparse-mode path in use (Euler): the fused one keeps the
-// brick-boundary planes and a row per listed cell (in FS_), the unfused one a
-// compact WENO staging for up to a quarter of the cells.
+// Buffers of the sparse-mode path in use (Euler), after a sync of the stream: the
+// fused one keeps the brick-boundary planes and a row per listed cell (in FS_),
+// the unfused one a compact WENO staging for up to a quarter of the cells.  Those
+// of the other path are given back (256^3: 3 GB and 4 GB), before the new ones are
+// taken; if that fails, evaluations are refused until a call here succeeds.
 void Solver::pathBuffers() {
   if (nv_ != 5) return;
   const size_t nc = size_t(ncell_), FQ = size_t(wts_.F) * wts_.Q;
   wsCap_ = int(std::max<size_t>(1, (nc + 3) / 4));
+  double *&unused = fusedNow() ? WS_ : SB_;
+  if (unused) {
+    check(hipFree(unused), "hipFree");
+    unused = nullptr;
+  }
   if (fusedNow() && !SB_) SB_ = dalloc<double>(surf_elems(cfg_.dim, cfg_.nQuad, grid_, sb_), "surface planes");
   if (!fusedNow() && !WS_) WS_ = dalloc<double>(size_t(wsCap_) * FQ * nv_, "compact WENO states");
 }
