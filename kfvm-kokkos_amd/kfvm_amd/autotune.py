@@ -7,8 +7,11 @@ size and records the fastest shape per size:
     python -m kfvm_amd.autotune [--sizes 64 128 256 512] [--problems 64] [--steps 4] [--out FILE]
 
 For each size and shape: a batch of `problems` four-quadrant problems (seeds
-0, 1, ...), two untimed steps, then `steps` timed steps with the per-kernel
-HIP-event timing; the flux kernel's milliseconds per launch decide.  With a
+0, 1, ...) with WENO on every cell, two untimed steps, then `steps` timed steps
+with the per-kernel HIP-event timing; the flux kernel's milliseconds per launch
+decide.  (The shapes are those of the flux kernel that reads every face state:
+full WENO, as after an unphysical step, GLM-MHD, linear advection and
+KFVM_FUSED=0.  The fused kernel of sparse Euler evaluations has one brick.)  With a
 fixed step the shapes give the same states bit for bit (only the brick tiling
 of the faces changes; with the adaptive controller the error norm's block
 partial sums regroup, a rounding-level difference), so the choice is a speed
@@ -49,7 +52,7 @@ def shape_for(n, table):
 def time_shape(n, shape, problems, steps, t_end=0.25):
     # a fixed step (the same stage sequence as the adaptive run): the states
     # of the shapes are then comparable bit for bit
-    text = quadrant_text(n, t_end) + f"tune:fluxbrick {shape}\ntime:fixeddt 1e-4\n"
+    text = quadrant_text(n, t_end, wenothresh=-1.0) + f"tune:fluxbrick {shape}\ntime:fixeddt 1e-4\n"
     s = kfvm_amd.Solver(init_text=text, seeds=list(range(problems)))
     for _ in range(2):
         s.take_step()
