@@ -136,6 +136,7 @@ void Solver::setup() {
   }
   grid_.rs = int(cfg_.rs);
 
+  check(hipGetDevice(&dev_), "hipGetDevice");
   check(hipStreamCreate(&stream_), "hipStreamCreate");
   const size_t nc = size_t(ncell_);
   const size_t FQ = size_t(wts_.F) * wts_.Q;
@@ -1304,8 +1305,6 @@ void Solver::copyToHost(void *dst, const void *src, size_t bytes) const {
     check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "copy to host");
     return;
   }
-  int dev = 0;
-  check(hipGetDevice(&dev), "hipGetDevice");
   std::lock_guard<std::mutex> lock(pinMutex_);  // one copy at a time uses the buffers
   if (!pin_ && hipHostMalloc((void **)&pin_, 8 * kChunk, hipHostMallocDefault) != hipSuccess) {
     pin_ = nullptr;
@@ -1316,7 +1315,9 @@ void Solver::copyToHost(void *dst, const void *src, size_t bytes) const {
   std::vector<hipError_t> err(nt, hipSuccess);
   std::vector<std::thread> th;
   auto work = [&](unsigned t) {
-    hipError_t e = hipSetDevice(dev);
+    int caller = dev_;  // kept: a share may run on the calling thread
+    (void)hipGetDevice(&caller);
+    hipError_t e = hipSetDevice(dev_);  // an event must be of its stream's device
     hipEvent_t ev = nullptr;
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     char *const buf = pin_ + t * kChunk;
@@ -1328,6 +1329,7 @@ void Solver::copyToHost(void *dst, const void *src, size_t bytes) const {
       if (e == hipSuccess) std::memcpy(static_cast<char *>(dst) + off, buf, n);
     }
     if (ev) (void)hipEventDestroy(ev);
+    if (caller != dev_) (void)hipSetDevice(caller);
     err[t] = e;
   };
   unsigned started = 0;

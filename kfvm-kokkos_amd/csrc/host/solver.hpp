@@ -157,6 +157,7 @@ class Solver {
   Grid grid_{};
   int nv_ = 5;
   int64_t ncell_ = 0;
+  int dev_ = 0;  // the GPU that was current when the solver was made
   hipStream_t stream_ = nullptr;
 
   // device buffers
