@@ -1,6 +1,8 @@
 """Device memory of the two sparse-mode paths: a 3D Euler solver that takes the
 learned selection gives the fused path's surface planes back and gets them again
 without it, and evaluates as a solver that never switched."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -10,14 +12,16 @@ pytestmark = pytest.mark.gpu
 
 
 def test_selection_keeps_one_path_s_buffers():
-    import torch
-
     import kfvm_amd
     from kfvm_amd import train_indicator
+    kfvm_amd.load_library()
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the library's own HIP runtime
 
     def free():
-        torch.cuda.synchronize()
-        return torch.cuda.mem_get_info()[0]
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
 
     n = (96, 80, 72)
     cells = n[0] * n[1] * n[2]
