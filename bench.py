@@ -347,7 +347,7 @@ def main():
     ap.add_argument("--threshold", type=float, default=0.0,
                     help="logit above which the learned indicator selects WENO")
     ap.add_argument("--fused", action="store_true",
-                    help="fused reconstruction + flux path (the flux kernel recomputes the linear states)")
+                    help="fused reconstruction + flux path where it is built (the default; KFVM_FUSED=0: unfused)")
     ap.add_argument("--cpu-workloads", type=int, default=0, metavar="N",
                     help="only time the CPU oracle: 64^3 to t = 0.2 and N^3 for 2 fixed-dt steps (no GPU)")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="MIB",

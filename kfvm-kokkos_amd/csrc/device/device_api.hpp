@@ -82,10 +82,8 @@ constexpr size_t kNoAllocScratchBytes = size_t(256) << 20;
 void *noalloc_scratch();
 
 // Learned WENO selection run by the Euler linear pass on its staged brick:
-// network parameters and the selection's inputs and outputs (those of
-// launch_learned_select).
+// network parameters and the selection's inputs and outputs.
 struct LearnArgs {
-  const double *eint = nullptr;     // per-cell internal energy (the limiter's plane)
   const double *theta = nullptr;    // positivity theta of the previous RHS
   const double *nadFlag = nullptr;  // cells that failed the last admissibility check
   const float *P = nullptr;         // network parameters (bfloat16 values)
@@ -139,7 +137,7 @@ hipError_t launch_cell_props(int dim, const double *U, double *props, const Grid
 // whose states violate a limiter bound are appended to ppList (count in
 // *ppCount, zeroed by the caller) and limited by launch_pp_lanes.
 // la (Euler, may be null): the learned WENO selection runs in the same kernel
-// on the staged brick (outputs those of launch_learned_select).
+// on the staged brick.
 // PW (Euler, may be null): the parity coefficients of the face points
 // (host/parity.hpp, [type][C]) of mirror-symmetric weights; without them
 // the dense products with W0T.
@@ -297,11 +295,12 @@ hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
 int net_inputs(int dim);  // features per cell
 int net_params(int dim);  // floats in the parameter vector
 int net_train_block();    // samples per training block
+// the learned selection of GLM-MHD runs (Euler: LearnArgs of the linear pass)
+hipError_t launch_learned_select(int dim, const double *U, const double *theta, const double *nadFlag,
+                                 const float *P, float thr, double *wflag, int *list,
+                                 int *counter, const Grid &g, int *pos, int cap, hipStream_t s);
 // eint: per-cell internal energy (the first plane of the limiter's cell
 // properties) for nv 5; unused for nv 9
-hipError_t launch_learned_select(int dim, int nv, const double *U, const double *eint, const double *theta,
-                                 const double *nadFlag, const float *P, float thr, double *wflag, int *list,
-                                 int *counter, const Grid &g, int *pos, int cap, hipStream_t s);
 hipError_t launch_features(int dim, int nv, const double *U, const double *eint, float *X, const Grid &g,
                            hipStream_t s);
 hipError_t launch_labels(int dim, int nq, int nv, const double *U, const double *FSL, const double *FSW, float tau,

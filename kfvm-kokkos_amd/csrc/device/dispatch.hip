@@ -205,11 +205,10 @@ int net_inputs(int dim) { return dim == 3 ? dev::Net<3>::NIN : dev::Net<2>::NIN;
 int net_params(int dim) { return dim == 3 ? dev::Net<3>::NP : dev::Net<2>::NP; }
 int net_train_block() { return dev::TB; }
 
-hipError_t launch_learned_select(int dim, int nv, const double *U, const double *eint, const double *theta,
-                                 const double *nadFlag, const float *P, float thr, double *wflag, int *list,
+hipError_t launch_learned_select(int dim, const double *U, const double *theta, const double *nadFlag,
+                                 const float *P, float thr, double *wflag, int *list,
                                  int *counter, const Grid &g, int *pos, int cap, hipStream_t s) {
-  if (nv != 5 && nv != 9) return hipErrorInvalidValue;
-  KFVM_SELECT(dim, 2, L::learned_select(nv, U, eint, theta, nadFlag, P, thr, wflag, list, counter, g, pos, cap, s));
+  KFVM_SELECT(dim, 2, L::learned_select(U, theta, nadFlag, P, thr, wflag, list, counter, g, pos, cap, s));
 }
 hipError_t launch_features(int dim, int nv, const double *U, const double *eint, float *X, const Grid &g,
                            hipStream_t s) {

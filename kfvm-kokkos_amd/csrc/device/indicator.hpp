@@ -159,7 +159,8 @@ constexpr int feature_lds(int k) {
          (D == 3 ? Bx::LX * Bx::LY * (ST.off[n][2] + Bx::H) : 0);
 }
 
-// Learned selection: WENO where the network's logit exceeds thr, where the
+// Learned selection of GLM-MHD runs (those of the Euler equations: learned_tail):
+// WENO where the network's logit exceeds thr, where the
 // previous RHS evaluation limited the cell (theta < 1, as the KXRCF selector),
 // or where the last step's admissibility check failed (nadFlag > 0).  One
 // block per brick of the linear reconstruction's geometry: rho and p of the
@@ -170,9 +171,8 @@ constexpr int feature_lds(int k) {
 // the B operand, layer 1 is 2 x ceil(NIN/32) x 3 MFMAs, layer 2 2 x 3 (its
 // K order follows layer 1's output layout, with W2's columns permuted to
 // match), and the last layer a dot product reduced over the four lane groups.
-template <int D, int NV>
+template <int D>
 __global__ __launch_bounds__(RBox<D>::NT) void k_learned_select(const double *__restrict__ U,
-                                                                const double *__restrict__ eint,
                                                                 const double *__restrict__ theta,
                                                                 const double *__restrict__ nadFlag,
                                                                 const float *__restrict__ P, float thr,
@@ -199,9 +199,9 @@ __global__ __launch_bounds__(RBox<D>::NT) void k_learned_select(const double *__
     const int gi = i0 + a - H, gj = j0 + bb - H, gk = D == 3 ? k0 + cz_ - H : k0;
     // box cells beyond the grid's far edges by more than the halo are never read
     if (gi < g.nx + H && gj < g.ny + H && (D == 2 || gk < g.nz + H)) {
-      const size_t q = map_cell<D, NV>(g, gi, gj, gk).idx;
+      const size_t q = map_cell<D, 9>(g, gi, gj, gk).idx;
       sr[idx] = U[q];
-      sp[idx] = gm1 * cell_eint<NV>(U, eint, q, g.ncell);
+      sp[idx] = gm1 * cell_eint<9>(U, nullptr, q, g.ncell);
     } else {
       sr[idx] = 0.0;
       sp[idx] = 0.0;

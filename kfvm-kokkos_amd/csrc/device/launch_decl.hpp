@@ -45,8 +45,8 @@ struct Launch {
   // ---- learned troubled-cell indicator
   // nv 5 (Euler; eint = the limiter's internal-energy plane) or 9 (GLM-MHD;
   // the internal energy comes from the conserved variables)
-  static hipError_t learned_select(int nv, const double *U, const double *eint, const double *theta,
-                                   const double *nadFlag, const float *P, float thr, double *wflag, int *list,
+  static hipError_t learned_select(const double *U, const double *theta, const double *nadFlag,
+                                   const float *P, float thr, double *wflag, int *list,
                                    int *counter, const Grid &g, int *pos, int cap, hipStream_t s);
   static hipError_t features(int nv, const double *U, const double *eint, float *X, const Grid &g, hipStream_t s);
   static hipError_t labels(int nv, const double *U, const double *FSL, const double *FSW, float tau, float *Y,

@@ -262,15 +262,11 @@ hipError_t LaunchMhd<D, NQ>::pp(const double *U, double *FS, double *SRC, double
 }
 
 template <int D, int NQ>
-hipError_t Launch<D, NQ>::learned_select(int nv, const double *U, const double *eint, const double *theta,
-                                         const double *nadFlag, const float *P, float thr, double *wflag, int *list,
+hipError_t Launch<D, NQ>::learned_select(const double *U, const double *theta, const double *nadFlag,
+                                         const float *P, float thr, double *wflag, int *list,
                                          int *counter, const Grid &g, int *pos, int cap, hipStream_t s) {
-  if (nv == 9)
-    hipLaunchKernelGGL((dev::k_learned_select<D, 9>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U, eint,
-                       theta, nadFlag, P, thr, wflag, list, counter, g, pos, cap);
-  else
-    hipLaunchKernelGGL((dev::k_learned_select<D, 5>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U, eint,
-                       theta, nadFlag, P, thr, wflag, list, counter, g, pos, cap);
+  hipLaunchKernelGGL((dev::k_learned_select<D>), dim3(bricks(g)), dim3(dev::RBox<D>::NT), 0, s, U, theta, nadFlag, P,
+                     thr, wflag, list, counter, g, pos, cap);
   return hipGetLastError();
 }
 

@@ -549,10 +549,13 @@ __device__ inline void mhd_pp_cell(const double *__restrict__ U, double *__restr
 // One thread per cell, so that the accesses of neighbouring listed cells to a
 // state plane share cache lines (a group of lanes per cell touches a line of
 // its own for every point and variable: 96^3, 13 % of the cells, 0.47 ms; this
-// form 0.44; what is left is the scattered lines of cells that are not all listed).  The pass that converts also makes the limiter's tests and the
+// form 0.44; what is left is the scattered lines of cells that are not all
+// listed).  The pass that converts also makes the limiter's tests and the
 // speeds: a cell inside every bound is done with it, the others go through the
-// exact sequence (mhd_pp_cell).  Waves are workgroups: short lists still
-// spread over the CUs.
+// exact sequence (mhd_pp_cell), which pays also where most cells do (64^3, all
+// listed, 64 % limited: WENO and this pass 2.41 ms with groups of lanes and the
+// dense WENO, 1.63 now).  Waves are workgroups: short lists still spread over the
+// CUs.
 template <int D, int NQ>
 __global__ __launch_bounds__(64) void k_mhd_weno_post(const double *__restrict__ U, double *__restrict__ FS,
                                                       double *__restrict__ SRC, Grid g,
@@ -643,10 +646,6 @@ __global__ __launch_bounds__(BLK) void k_mhd_pp(const double *__restrict__ U, do
 }
 
 // ------------------------------------------------------------ cleaning speed
-__device__ inline double glm_ch(const unsigned long long *chBits) {
-  return __longlong_as_double((long long)chBits[0]) - __longlong_as_double((long long)chBits[1]);
-}
-
 // -------------------------------------------------------------- GLM sources
 // Source terms (SourceTerms_K, MHD_GLM_K.H:316-547; no user forcing for the
 // registry problems) of cell c at its NQ^D interior points, integrated into

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(BLK) void k_flux_points(const double *__restrict__ 
     const bool lBrick = (dir == 0 ? fi > 0 : (dir == 1 ? fj > 0 : fk > 0)) && lIn;
     const bool needed = rBrick || lBrick;
     // the side's source; a cell off the grid along dir wraps (periodic) or
-    // mirrors the other side (wall), as face_state resolves it
+    // mirrors the other side (wall)
     auto source = [&](int x, int y, int z) {
       const int n_ax = dir == 0 ? g.nx : (dir == 1 ? g.ny : g.nz);
       int pos = dir == 0 ? x : (dir == 1 ? y : z);

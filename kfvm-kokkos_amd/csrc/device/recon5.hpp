@@ -132,8 +132,9 @@ __device__ void learned_tail(double *lds, const LearnArgs &la, const Grid &g, in
 // points stay in registers until the energy completes them, which gives
 // p/rho^gamma and the limiter's fast test without reading the states back.
 //
-// Used with weight tables that are not mirror-symmetric (set by the caller);
-// the symmetric tables run k_linear_par.
+// Used by 3D runs with the learned selection, whose choice of cells reads the
+// order of these sums (points5.hpp), and with weight tables that are not mirror-
+// symmetric (set by the caller); all others run k_linear_par.
 //
 // LEARN = true: the learned WENO selection follows on the same brick
 // (learned_tail), in place of a separate selection kernel that would stage

@@ -712,49 +712,6 @@ struct Brick {
   static constexpr int PXF = pad64(NXF), PYF = pad64(NYF), PZF = pad64(NZF), PF = PXF + PYF + PZF;
 };
 
-// Face state of cell (ci,cj,ck) on its face f at point q; cells outside the
-// domain resolve through periodic wrap or the face boundary condition (copy of
-// the inner state, with the mirror's sign for reflecting / noslip walls).
-// row >= 0 (Euler): the cell's states are row `row` of the compact WENO
-// staging ws[t][F*Q*5] instead of its FS slots.
-template <int D, int NQ, int NV>
-__device__ inline void face_state(const double *__restrict__ FS, const Grid &g, int ci, int cj,
-                                  int ck, int f, int q, const double *inner, double *out, int row = -1,
-                                  const double *__restrict__ ws = nullptr) {
-  constexpr int Q = Shape<D, NQ>::Q;
-  const int ax = f >> 1;
-  const int n_ax = ax == 0 ? g.nx : (ax == 1 ? g.ny : g.nz);
-  int pos = ax == 0 ? ci : (ax == 1 ? cj : ck);
-  if (pos < 0 || pos >= n_ax) {
-    const bool low = pos < 0;
-    const int bcLo = ax == 0 ? g.bc[0] : (ax == 1 ? g.bc[2] : g.bc[4]);
-    const int bcHi = ax == 0 ? g.bc[1] : (ax == 1 ? g.bc[3] : g.bc[5]);
-    if ((low ? bcLo : bcHi) != 0) {
-      const unsigned mLo = ax == 0 ? g.negmask[0] : (ax == 1 ? g.negmask[2] : g.negmask[4]);
-      const unsigned mHi = ax == 0 ? g.negmask[1] : (ax == 1 ? g.negmask[3] : g.negmask[5]);
-      const unsigned m = NV >= 5 ? (low ? mLo : mHi) : 0u;
-#pragma unroll
-      for (int v = 0; v < NV; v++) out[v] = ((m >> v) & 1u) ? -inner[v] : inner[v];
-      return;
-    }
-    pos = pos < 0 ? pos + n_ax : pos - n_ax;
-    if (ax == 0) ci = pos;
-    else if (ax == 1) cj = pos;
-    else ck = pos;
-  }
-  const size_t cell = (size_t(ck) * g.ny + cj) * g.nx + ci;
-  const size_t nc = g.ncell;
-  if (NV == 5 && row >= 0) {
-    const double *r = ws + size_t(row) * (Shape<D, NQ>::F * Q * 5) + (f * Q + q) * 5;
-#pragma unroll
-    for (int v = 0; v < NV; v++) out[v] = r[v];
-    return;
-  }
-#pragma unroll
-  for (int v = 0; v < NV; v++)
-    out[v] = FS[fs_base(cell, Shape<D, NQ>::F * Q * NV) + (size_t(f * Q + q) * NV + v) * FSB];
-}
-
 // GLM-MHD source terms of one cell integrated into rhs (defined with the
 // GLM-MHD kernels).
 template <int D, int NQ>
@@ -876,7 +833,7 @@ __global__ __launch_bounds__(BLK, NV == 9 ? (D == 3 && NQ == 3 ? 1 : 2) : 3) voi
     const bool lBrick = (dir == 0 ? fi > 0 : (dir == 1 ? fj > 0 : fk > 0)) && lIn;
     const bool needed = rBrick || lBrick;
     // the side's source; a cell off the grid along dir wraps (periodic) or
-    // mirrors the other side (wall), as face_state resolves it
+    // mirrors the other side (wall)
     auto source = [&](int x, int y, int z) {
       const int n_ax = dir == 0 ? g.nx : (dir == 1 ? g.ny : g.nz);
       int pos = dir == 0 ? x : (dir == 1 ? y : z);

@@ -695,7 +695,7 @@ void Solver::pipelineMhd(const double *Uin, const RKArgs &a0) {
     });
     if (lrn) {
       timed("select", [&] {
-        return launch_learned_select(dim, 9, Uin, nullptr, thPrev, nadFlag_, netP_, netThr_, wflag_, list_,
+        return launch_learned_select(dim, Uin, thPrev, nadFlag_, netP_, netThr_, wflag_, list_,
                                      counter_, grid_, nullptr, 0, stream_);
       });
     } else {
@@ -753,7 +753,6 @@ void Solver::pipeline(const double *Uin, const RKArgs &a) {
   double *wi = lrn ? nullptr : WI_;
   LearnArgs la;
   if (lrn) {
-    la.eint = props_;
     la.theta = thPrev;
     la.nadFlag = nadFlag_;
     la.P = netP_;
