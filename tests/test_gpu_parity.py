@@ -58,6 +58,8 @@ CASES = {
                                               rk="threestarp", fixeddt=0.004),
     "quadrant2d_sparse": config(dim=2, n=(48, 40, 1), problem="quadrant2d", seed=7, user=(),
                                 fixeddt=0.002),
+    "quadrant2d_nq3_sparse": config(dim=2, n=(37, 42, 1), nq=3, problem="quadrant2d", seed=5, user=(),
+                                    bc="periodic", fixeddt=0.002),
     "quadrant2d_full_nq3": config(dim=2, n=(32, 32, 1), nq=3, problem="quadrant2d", seed=3,
                                   user=(), wenothresh=-1.0, fixeddt=0.002),
     "shear2d_periodic": config(dim=2, n=(48, 48, 1), problem="shear2d", seed=1, user=(),
@@ -171,7 +173,8 @@ def test_unphysical_rejection_forces_full_weno():
     assert r.max() <= 1e-10
 
 
-FUSED_CASES = ["riemann3d_sparse", "riemann3d_periodic_nq3_sparse", "quadrant2d_sparse", "shear2d_periodic",
+# both face rules in 2D, the 2x2 rule in 3D (the 3x3 rule has no fused path)
+FUSED_CASES = ["riemann3d_sparse", "quadrant2d_sparse", "quadrant2d_nq3_sparse", "shear2d_periodic",
                "riemann3d_hll_reflect", "riemann3d_llf_noslip_threestar"]
 
 
@@ -197,21 +200,38 @@ def test_fused_path_equals_unfused_path(name, monkeypatch):
     assert np.array_equal(fus.flags, ref.flags)
 
 
-@pytest.mark.parametrize("name", ["riemann3d_sparse", "riemann3d_full", "riemann3d_hll_reflect"])
+# 3D NQ=2 runs of the matrix-core WENO kernel: WENO on every cell, and lists of
+# KXRCF cells with derivative tables that lack the mirror symmetry (the symmetric
+# ones run k_weno_par): with a row for every listed cell (the fused path), and
+# with the compact staging of a quarter of the cells, which one list fits and the
+# other exceeds
+MATRIX_CASES = {
+    "full": (CASES["riemann3d_full"], "1"),
+    "rows": (CASES["riemann3d_sparse"], "1"),
+    "rows_reflect": (CASES["riemann3d_hll_reflect"], "1"),
+    "staging": (CASES["riemann3d_sparse"], "0"),
+    "staging_exceeded": (dict(CASES["riemann3d_sparse"], n=(13, 12, 11)), "0"),
+}
+
+
+@pytest.mark.parametrize("name", sorted(MATRIX_CASES))
 def test_matrix_core_weno_matches_scalar_weno(name, monkeypatch):
-    """3D NQ=2 runs KFVM-WENO on the FP64 matrix cores (k_wenorec5_mfma); the
-    scalar kernel (KFVM_WENO_SCALAR=1) sums the same products in the
-    reference's order.  Three fixed-dt steps of each, every launch of one run
+    """k_wenorec5_mfma (FP64 matrix cores) against the scalar kernel
+    (KFVM_WENO_SCALAR=1), which sums the same products in the reference's
+    order.  Three fixed-dt steps of each, every launch of one run
     on the matrix cores and of the other on the scalar kernel, agree to
     rounding (per-cell relative difference <= 1e-13) with the same WENO
     flags; the limiter's theta, computed from the WENO states, to 1e-12."""
     import kfvm_amd
-    c = CASES[name]
+    c, fused = MATRIX_CASES[name]
     text = init_text(c)
-    monkeypatch.setenv("KFVM_WENO_SCALAR", "1")
-    ref = kfvm_amd.Solver(init_text=text)
-    monkeypatch.setenv("KFVM_WENO_SCALAR", "0")
-    mat = kfvm_amd.Solver(init_text=text)
+    monkeypatch.setenv("KFVM_FUSED", fused)
+    ref, mat = kfvm_amd.Solver(init_text=text), kfvm_amd.Solver(init_text=text)
+    if name != "full":
+        f, d = mat.weights
+        d[0, 0, 1] += 1e-9
+        for s in (ref, mat):
+            s.set_weights(f, d)
     for _ in range(3):
         monkeypatch.setenv("KFVM_WENO_SCALAR", "1")
         assert ref.take_step() == 0
@@ -223,7 +243,49 @@ def test_matrix_core_weno_matches_scalar_weno(name, monkeypatch):
     dth = np.abs(fm[1] - fr[1]).max()
     print(f"[weno] {name}: matrix-core vs scalar WENO max cell rel diff {r.max():.3e}, max |d theta| "
           f"{dth:.3e}, WENO cells {nw}", flush=True)
-    assert nw > 0
+    # lists: a last group of 16 cells that is not whole, and the staging as named
+    cells = fm[0].size
+    assert nw == cells if name == "full" else (0 < nw < cells and nw % 16 != 0)
+    if fused == "0":
+        assert (nw > (cells + 3) // 4) == (name == "staging_exceeded")
     assert r.max() <= 1e-13
     assert np.array_equal(fm[0], fr[0])
     assert dth <= 1e-12
+
+
+def test_matrix_core_weno_of_the_learned_selection(monkeypatch):
+    """The matrix-core kernel on the cells a network picks (the symmetric tables
+    keep it there), against the scalar kernel: right-hand sides of one state
+    without constant regions, whose lists are therefore the same, within 1e-12 of
+    the largest value."""
+    import indicator_ref as ir
+
+    import kfvm_amd
+    c = config(n=(18, 15, 13), bc="periodic")
+    text = init_text(c)
+    rng = np.random.default_rng(4)
+    P = rng.normal(0.0, 0.4, ir.net_sizes(3)[1]).astype(np.float32)
+    P[-1] = 0.3
+    K, F = [], []
+    for scalar in ("1", "0"):
+        monkeypatch.setenv("KFVM_WENO_SCALAR", scalar)
+        s = kfvm_amd.Solver(init_text=text)
+        x, y, z = (2.0 * np.pi * (np.arange(m) + 0.5) / m for m in c["n"])
+        a = np.sin(x)[None, None, :] + np.sin(2.0 * y)[None, :, None] + np.cos(z)[:, None, None]
+        b = np.cos(2.0 * x)[None, None, :] + np.sin(y)[None, :, None] + np.sin(2.0 * z)[:, None, None]
+        rho, p, vel = 1.0 + 0.2 * a, 1.0 + 0.2 * b, (0.3 * a, 0.2 * b, 0.1 * (a + b))
+        s.state = np.stack([rho] + [rho * v for v in vel] +
+                           [p / (c["gamma"] - 1.0) + 0.5 * rho * sum(v * v for v in vel)])
+        fl = np.zeros((2,) + s.shape[1:])
+        fl[1] = 1.0
+        s.flags = fl
+        s.set_indicator(kfvm_amd.float_to_bf16(P), 0.0)
+        s.eval_rhs()
+        K.append(s.rhs)
+        F.append(s.flags[0])
+    n, cells = int(F[0].sum()), F[0].size
+    r = np.abs(K[1] - K[0]).max() / np.abs(K[0]).max()
+    print(f"[weno] learned: matrix-core vs scalar WENO {r:.3e}, {n} of {cells} cells", flush=True)
+    assert np.array_equal(F[0], F[1])
+    assert 0 < n < cells and n % 16 != 0
+    assert r <= 1e-12
