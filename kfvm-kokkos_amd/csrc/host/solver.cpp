@@ -1299,7 +1299,9 @@ void Solver::copyToHost(void *dst, const void *src, size_t bytes) const {
   check(hipStreamSynchronize(stream_), "sync");
   constexpr size_t kChunk = size_t(2) << 20;
   const size_t chunks = (bytes + kChunk - 1) / kChunk;
-  const unsigned nt = unsigned(std::min<size_t>({size_t(8), chunks / 4, size_t(std::thread::hardware_concurrency())}));
+  // (the number of processors is a system call of a few us, as long as a small copy)
+  const unsigned nt =
+      chunks < 8 ? 1 : unsigned(std::min<size_t>({size_t(8), chunks / 4, size_t(std::thread::hardware_concurrency())}));
   if (nt < 2) {
     check(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost), "copy to host");
     return;
