@@ -156,16 +156,17 @@ struct Hydro {
   // HLLC with the low-Mach / shear corrections (Hydro_Riemann.H:97-187).  The
   // formulas are the reference's, arranged for few divisions and square roots,
   // which are most of the solver's time (each takes 8 to 16 issue slots):
-  //   - a common denominator is inverted once; 1/rho of both sides comes from
-  //     the reciprocal of their product;
+  //   - a common denominator is inverted once;
   //   - the larger of |v_L|/a_L and |v_R|/a_R is picked by its square, so M takes
   //     one reciprocal square root instead of two roots and two divisions;
-  //     products beyond the exponent range (velocities near 1e-160, densities
-  //     near 1e-155) take the separate operations (the tests cost 0.5 % of a pass);
+  //     products beyond the exponent range (velocities near 1e-160, speeds near
+  //     1e78) take the separate operations (the branch costs 0.1 to 0.8 % of a
+  //     pass; one more for the densities, inverted through their product, cost
+  //     0.3 % more than their two reciprocals here);
   //   - the star state is formed on the side the face lies on only;
   //   - the pressure ratio enters the power without being divided out
   //     (pow_ratio).
-  // 4 reciprocals, 2 quotients and 7 roots, against 5, 6 and 8 in solve_hllc_pt.
+  // 5 reciprocals, 2 quotients and 7 roots, against 5, 6 and 8 in solve_hllc_pt.
   // Results differ from the reference's by rounding only.
   template <int DIR>
   __device__ static inline double solve_hllc(double g, const double *uL, const double *uR,
@@ -173,16 +174,7 @@ struct Hydro {
     constexpr int v0 = 1 + DIR, v1 = 1 + (DIR + 1) % 3, v2 = 1 + (DIR + 2) % 3;
     const double gm1 = g - 1.0;
     const double rhoL = uL[0], rhoR = uR[0];
-    const double rho2 = rhoL * rhoR;
-    double irL, irR;
-    if (in_range(rho2)) {
-      const double ir = rcp_n(rho2);
-      irL = ir * rhoR;
-      irR = ir * rhoL;
-    } else {
-      irL = rcp_n(rhoL);
-      irR = rcp_n(rhoR);
-    }
+    const double irL = rcp_n(rhoL), irR = rcp_n(rhoR);
     const double unL = uL[v0] * irL, vtL = uL[v1] * irL, wtL = uL[v2] * irL;
     const double unR = uR[v0] * irR, vtR = uR[v1] * irR, wtR = uR[v2] * irR;
     const double vsqL = unL * unL + vtL * vtL + wtL * wtL, vsqR = unR * unR + vtR * vtR + wtR * wtR;
